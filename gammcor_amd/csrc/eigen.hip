@@ -805,6 +805,8 @@ __global__ __launch_bounds__(SY_THREADS) void sytrd_panel_kernel(PanelArgs<T> g)
     }
 }
 
+#include "sytrd_resident.hpp"
+
 // After the last panel: d[n-1], and clear everything on/above the diagonal so
 // the strictly lower triangle holds the unit-lower reflectors.
 template <class T>
@@ -1563,6 +1565,8 @@ static int eig_plan_host(int n, int batch, EigPlan<T>* p, std::vector<std::vecto
         if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
             ncu = prop.multiProcessorCount;
     }
+    p->ncu = ncu;
+    p->mres = res_max(batch, ncu);
     const int nblk = (n + 63) / 64;
     p->G = std::max(1, std::min(nblk, ncu / batch));
     GMC_CHECK(batch <= ncu, "eig_plan: batch %d exceeds the %d co-resident problems", batch, ncu);
@@ -1797,6 +1801,25 @@ int syevd_batched(hipStream_t s, EigPlan<T>& p, T* A, T* w)
         if (!capturing(s)) GMC_HIP(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         unsigned epoch = 0;
         for (int k = 0; k < n - 1; k += nb) {
+            if (n - k <= p.mres) {
+                // the rest fits in the register files: one resident launch,
+                // 3-5 us per column where a panel's column takes 15 or more
+                // (its two group barriers) at every order that fits
+                const int m = n - k;
+                const ResShape rs = res_shape(m, B, p.ncu);
+                const size_t words = (size_t)B * 2 * m * res_words<T>() * 2;   // of 32 bits
+                GMC_CHECK(rs.R > 0 && words * 4 <= (size_t)B * n * 3 * nb * sizeof(T), "syevd: resident shape");
+                ResArgs<T> ra{A, p.d, p.e, p.tau, reinterpret_cast<unsigned long long*>(p.X), p.err, n, k, rs.G};
+                void* rargs[] = {&ra};
+                const void* rk = res_kernel<T>(rs.R, rs.C);
+                const size_t rl = res_lds<T>(m, rs.R);
+                if (!capturing(s)) GMC_HIP(hipFuncSetAttribute(rk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)rl));
+                hipLaunchKernelGGL(zero_u32, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s,
+                                   reinterpret_cast<unsigned*>(p.X), (int)words);
+                ProfScope ps(s, sizeof(T) == 8 ? "sytrd_resident_f64" : "sytrd_resident_f32", 0.0);
+                GMC_TRY(launch_persistent(rk, dim3(B * rs.G), dim3(rs.NT), rargs, rl, s));
+                break;
+            }
             const int kb = std::min(nb, n - 1 - k);
             const int vec = (n % (16 / (int)sizeof(T)) == 0) && (reinterpret_cast<uintptr_t>(A) % 16 == 0) &&
                             (reinterpret_cast<uintptr_t>(p.vg) % 16 == 0);

@@ -31,6 +31,8 @@ struct EigPlan {
     int nb = 32;            // tridiagonalisation panel width
     int nbb = 128;          // back-transformation block width (<= 256 in FP32, 128 in FP64)
     int G = 1;              // workgroups cooperating on one problem
+    int ncu = 0;            // compute units of the device
+    int mres = 0;           // largest trailing order the resident reduction takes (sytrd_resident.hpp)
     std::vector<DcLevel> levels;
     unsigned char* d_split = nullptr;   // split flags (n)
     size_t ws_bytes = 0;
