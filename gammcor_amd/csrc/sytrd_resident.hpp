@@ -28,7 +28,7 @@
 // 3.3 us per column at order 410, about half of it the exchange; the FP64
 // update and product of R C elements per thread are most of the rest at 2048.
 //
-// Included by eigen.hip only (wave_sum, wave_sum_cols, ilog2).
+// Included by eigen.hip only, inside its namespace.
 #pragma once
 
 constexpr int RES_THREADS = 512, RES_WAVES = RES_THREADS / 64;
@@ -69,100 +69,6 @@ __device__ inline void res_unpack(const unsigned long long (&x)[4], double& w, d
     w = __longlong_as_double((long long)((x[1] << 32) | (x[0] & 0xffffffffull)));
     a = __longlong_as_double((long long)((x[3] << 32) | (x[2] & 0xffffffffull)));
 }
-__device__ inline float read_lane(float v, int l)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-__device__ inline double read_lane(double v, int l)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffff), l);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
-// ---- sums over a wave on the DPP and lane-swap paths (the LDS-crossbar
-// shuffles take several times their latency, and every sum here is on the
-// column's critical path)
-template <int CTRL>
-__device__ inline float dpp_mov(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
-template <int CTRL>
-__device__ inline double dpp_mov(double v)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffff), CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140;
-// a + b after a's upper half (32 lanes; or a's odd rows of 16, O = 16) and
-// b's lower half (even rows) have changed places: the lower lanes get the sum
-// of a over both halves, the upper ones that of b
-template <int O>
-__device__ inline float swap_add(float a, float b)
-{
-    const auto r = O == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false)
-                           : __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-template <int O>
-__device__ inline double swap_add(double a, double b)
-{
-    const unsigned long long x = (unsigned long long)__double_as_longlong(a), y = (unsigned long long)__double_as_longlong(b);
-    const auto lo = O == 32 ? __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false)
-                            : __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
-    const auto hi = O == 32 ? __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false)
-                            : __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
-    return __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])) +
-           __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
-}
-// The sum of v over the wave, in every lane.
-template <class T>
-__device__ inline T res_wave_sum(T v)
-{
-    v += dpp_mov<DPP_XOR1>(v);
-    v += dpp_mov<DPP_XOR2>(v);
-    v += dpp_mov<DPP_HALF_MIRROR>(v);
-    v += dpp_mov<DPP_MIRROR>(v);
-    v = swap_add<16>(v, v);
-    return swap_add<32>(v, v);
-}
-// One halving step across lane bit O: a lane keeps H of its values and adds
-// its partner's share of them; below one value per lane plain sums.
-template <int H, int O, int CTRL, int KV, class T>
-__device__ inline void res_half(T (&s)[KV], int lane)
-{
-    if constexpr (H >= 1) {
-        const bool up = (lane & O) != 0;
-#pragma unroll
-        for (int k = 0; k < H; k++) {
-            const T send = up ? s[k] : s[k + H], keep = up ? s[k + H] : s[k];
-            s[k] = keep + dpp_mov<CTRL>(send);
-        }
-    } else {
-        s[0] += dpp_mov<CTRL>(s[0]);
-    }
-}
-// The sums over the wave of KV values per lane (KV = 8 or 16): the lane gets
-// that of column lane >> (6 - log2 KV).
-template <int KV, class T>
-__device__ inline T res_sum_cols(T (&s)[KV], int lane)
-{
-    static_assert(KV == 8 || KV == 16, "columns per reduction");
-#pragma unroll
-    for (int k = 0; k < KV / 2; k++) s[k] = swap_add<32>(s[k], s[k + KV / 2]);
-#pragma unroll
-    for (int k = 0; k < KV / 4; k++) s[k] = swap_add<16>(s[k], s[k + KV / 4]);
-    res_half<KV / 8, 8, DPP_MIRROR>(s, lane);
-    res_half<KV / 16, 4, DPP_HALF_MIRROR>(s, lane);
-    res_half<0, 2, DPP_XOR2>(s, lane);
-    res_half<0, 1, DPP_XOR1>(s, lane);
-    return s[0];
-}
-
 // Dynamic LDS of the kernel for a trailing order m.
 template <class T>
 constexpr size_t res_lds(int m, int R) { return ((size_t)m + 2 * RES_WAVES + 4 + 2 * R + (size_t)RES_WAVES * R) * sizeof(T); }
@@ -256,7 +162,7 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
                 }
                 s1 += wc[k] * v[k];
             }
-            s1 = res_wave_sum(s1);
+            s1 = wave_total(s1);
             if (lane == 0) redA[wave] = s1;
             __syncthreads();
             s1 = T(0);
@@ -311,11 +217,11 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
 #pragma unroll
                     for (int q = 0; q < CH; q++) acol[q0 + q] = a[q0 + q][k];
                 }
-            const T s = res_sum_cols<CH>(acc, lane);
+            const T s = wave_col_sums<CH>(acc, lane);
             constexpr int SH = 6 - ilog2<CH>();
             if ((lane & ((1 << SH) - 1)) == 0) part[wave * R + q0 + (lane >> SH)] = s;
         }
-        nrm = res_wave_sum(nrm);
+        nrm = wave_total(nrm);
         if (lane == 0) redB[wave] = nrm;
         __syncthreads();
         // the reflector
