@@ -43,7 +43,7 @@ struct EigPlan {
     T *dsort = nullptr, *zsort = nullptr, *dK = nullptr, *zK = nullptr, *taus = nullptr, *zh = nullptr;
     T *EV = nullptr, *rotc = nullptr, *rots = nullptr, *Tf = nullptr;
     int *perm = nullptr, *lst = nullptr, *lstD = nullptr, *org = nullptr, *rank = nullptr;
-    int *rotp = nullptr, *rotj = nullptr, *kcnt = nullptr, *rcnt = nullptr;
+    int *rotp = nullptr, *rotj = nullptr, *kcnt = nullptr;
     int *kpos = nullptr, *kc1 = nullptr, *kc2 = nullptr;   // merge GEMM column grouping
     unsigned* bar = nullptr;
     int* err = nullptr;
