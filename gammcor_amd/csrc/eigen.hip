@@ -831,60 +831,127 @@ __global__ void clear_upper_kernel(T* A, int n)
 }
 
 // ====================================================================== ormtr
-// T factor (upper triangular, ld nbb) of H(k)...H(k+kb-1) = I - V T V^T from
-// the Gram matrix Gm = V^T V (ld nbb) and tau: column i of T is
-// -tau_i T(0:i, 0:i) G(0:i, i), diagonal tau_i.  T lives in LDS as its
-// upper triangle packed by columns (column c at c (c + 1) / 2); column i of
-// G is read into LDS at step i, with tau (dynamic LDS: kb (kb + 1) / 2 + 2 kb
-// elements).  Workgroup (p, q) forms the factor of problem p's block
-// k = k0 + q nbb (kb = min(nbb, nu - 1 - k)): Gram matrix and factor at
-// (q B + p) nbb^2, so one launch can form every block's factor of a
-// back-transformation.
+// The block reflector of columns k .. k+kb-1 is I - V T V^T; every block's V,
+// and so its T and U = V T, are known before the back-transformation starts.
+// They are formed ahead in three launches over all blocks (Gram matrices, T
+// factors, U), so a block of the loop is two products: QK = V^T Z and
+// Z -= U QK.  (Per block launches with a T product in the loop: 31 + 31 us
+// per block of order 1281 on top of the two large products.)
 template <class T>
 constexpr int bt_max() { return sizeof(T) == 4 ? 256 : 128; }   // largest back-transformation block
+constexpr int LT = 128;        // largest triangle one workgroup inverts in LDS
+constexpr int LT_BASE = 16;    // its base triangles
+
+// Gram matrices G_q = V_q^T V_q (ld nbb, at (q B + p) nbb^2) of problem p's
+// blocks q: one workgroup per 64 x 64 tile on or above the diagonal.  V has
+// ld nu and unit diagonal, block q starts at column q nbb, row q nbb + 1.
 template <class T>
-__global__ __launch_bounds__(256) void larft_kernel(const T* Gm, const T* tau, T* Tf, int n, int nu, int k0, int nbb)
+__global__ __launch_bounds__(256) void bt_gram_kernel(const T* A, T* G, int nu, int nbb, int B)
+{
+    const int q = blockIdx.y, p = blockIdx.z;
+    const int k = q * nbb, kb = min(nbb, nu - 1 - k), m = nu - k - 1;
+    int tj, ti;
+    lower_tile(blockIdx.x, tj, ti);   // tj >= ti
+    if (ti * BM >= kb || tj * BN >= kb) return;
+    const T* V = A + (size_t)p * nu * nu + (k + 1) + (size_t)k * nu;
+    GemmShape g{kb, kb, m, true, false, (int64_t)nu, (int64_t)nu, (int64_t)nbb, 0, 0, 0, 1, 0};
+    gemm_tile<T, GemmBK<T>::value>(g, ti * BM, tj * BN, T(1), V, V, T(0), G + ((size_t)q * B + p) * nbb * nbb);
+}
+
+// T factor of a block (or of the 128-column part `blockIdx.z` of one) in
+// place of its Gram matrix: T^-1 = D^-1 + U with D = diag(tau) and U the
+// strict upper triangle of G, so T is an inverse of triangles: base triangles
+// of 16 by the column recurrence (column i of T is -tau_i T(0:i, 0:i)
+// G(0:i, i), diagonal tau_i), then T12 = -T1 U12 T2 from 16 to 32, 64, 128,
+// all in LDS.  The recurrence over 128 columns took 235 us at any order, its
+// serial chain of barriers; this takes about 20.
+template <class T>
+__global__ __launch_bounds__(256) void larft_kernel(T* G, const T* tau, int n, int nu, int nbb)
 {
     extern __shared__ char smem[];
-    const int p = blockIdx.x, q = blockIdx.y;
-    const int k = k0 + q * nbb, kb = min(nbb, nu - 1 - k);
-    const size_t at0 = ((size_t)q * gridDim.x + p) * nbb * nbb;
-    const T* G = Gm + at0;
-    T* Tm = Tf + at0;
-    const int tri = kb * (kb + 1) / 2;
-    T* t = reinterpret_cast<T*>(smem);
-    T* gcol = t + tri;
-    T* ts = gcol + kb;
-    for (int i = threadIdx.x; i < kb; i += 256) ts[i] = tau[(size_t)p * n + k + i];
-    for (int i = 0; i < kb; i++) {
-        const int ci = i * (i + 1) / 2;
-        for (int c = threadIdx.x; c < i; c += 256) gcol[c] = G[c + (size_t)i * nbb];
-        __syncthreads();
-        if ((int)threadIdx.x < i) {
-            const int c = threadIdx.x;
-            // four independent terms per pass keep LDS loads in flight
-            T acc0 = 0, acc1 = 0, acc2 = 0, acc3 = 0;
-            int c2 = c, at = c * (c + 1) / 2 + c;   // at = position of t(c, c2)
-            for (; c2 + 3 < i; c2 += 4) {
-                acc0 += t[at] * gcol[c2];
-                acc1 += t[at + c2 + 1] * gcol[c2 + 1];
-                acc2 += t[at + 2 * c2 + 3] * gcol[c2 + 2];
-                acc3 += t[at + 3 * c2 + 6] * gcol[c2 + 3];
-                at += 4 * c2 + 10;
+    T* t = reinterpret_cast<T*>(smem);   // LT x LT, column-major
+    T* ts = t + LT * LT;                 // LT
+    const int p = blockIdx.x, q = blockIdx.y, o = blockIdx.z * LT, tid = threadIdx.x;
+    const int k = q * nbb, kb = min(min(nbb, nu - 1 - k) - o, LT);   // columns of this triangle
+    if (kb <= 0) return;
+    T* Gb = G + ((size_t)q * gridDim.x + p) * nbb * nbb + o + (size_t)o * nbb;
+    for (int idx = tid; idx < LT * LT; idx += 256) {
+        const int r = idx % LT, c = idx / LT;
+        t[idx] = (r < c && c < kb) ? Gb[r + (size_t)c * nbb] : T(0);
+    }
+    if (tid < LT) ts[tid] = tid < kb ? tau[(size_t)p * n + k + o + tid] : T(0);
+    __syncthreads();
+    {
+        // thread (base triangle, row), in step over the columns
+        const int bt = tid / LT_BASE, r = tid % LT_BASE;
+        T* tb = t + (bt * LT_BASE) * (LT + 1);
+        const bool on = tid < LT;
+        for (int i = 0; i < LT_BASE; i++) {
+            T acc = 0;
+            if (on && r < i)
+                for (int c = r; c < i; c++) acc += tb[r + c * LT] * tb[c + i * LT];
+            __syncthreads();
+            if (on) {
+                const T ti = ts[bt * LT_BASE + i];
+                if (r < i) tb[r + i * LT] = -ti * acc;
+                if (r == i) tb[r + i * LT] = ti;
             }
-            for (; c2 < i; c2++) {
-                acc0 += t[at] * gcol[c2];
-                at += c2 + 1;
-            }
-            t[ci + c] = -ts[i] * ((acc0 + acc1) + (acc2 + acc3));
+            __syncthreads();
         }
-        if (threadIdx.x == 0) t[ci + i] = ts[i];
-        __syncthreads();
     }
-    for (int idx = threadIdx.x; idx < nbb * nbb; idx += 256) {
-        const int r = idx % nbb, c = idx / nbb;
-        Tm[idx] = (c < kb && r <= c) ? t[c * (c + 1) / 2 + r] : T(0);
+    for (int h = LT_BASE; h < LT && h < kb; h *= 2) {
+        // pairs of triangles T1 at d, T2 at d + h: W = U12 T2 into the unused
+        // block below the diagonal, then T12 = -T1 W
+        const int nout = LT / 2 * h;   // outputs over all pairs
+        for (int pass = 0; pass < 2; pass++) {
+            for (int idx = tid; idx < nout / 4; idx += 256) {
+                const int e = idx * 4, d = e / (h * h) * 2 * h, x = e % (h * h), r = x % h, c = x / h;
+                T acc[4] = {T(0), T(0), T(0), T(0)};
+                if (pass == 0) {
+                    // W(r, c) = sum_{l <= c} U12(r, l) T2(l, c)
+                    for (int l = 0; l <= c; l++) {
+                        const T y = t[d + h + l + (d + h + c) * LT];
+                        const T* u = t + d + r + (d + h + l) * LT;
+#pragma unroll
+                        for (int z = 0; z < 4; z++) acc[z] += u[z] * y;
+                    }
+                } else {
+                    // T12(r, c) = -sum_{l >= r} T1(r, l) W(l, c)
+                    for (int l = r; l < h; l++) {
+                        const T y = t[d + h + l + (d + c) * LT];
+                        const T* u = t + d + r + (d + l) * LT;
+#pragma unroll
+                        for (int z = 0; z < 4; z++) acc[z] += (l >= r + z ? u[z] : T(0)) * y;
+                    }
+                }
+#pragma unroll
+                for (int z = 0; z < 4; z++) {
+                    if (pass == 0) t[d + h + r + z + (d + c) * LT] = acc[z];
+                    else t[d + r + z + (d + h + c) * LT] = -acc[z];
+                }
+            }
+            __syncthreads();
+        }
     }
+    for (int idx = tid; idx < LT * LT; idx += 256) {
+        const int r = idx % LT, c = idx / LT;
+        if (r < kb && c < kb) Gb[r + (size_t)c * nbb] = r <= c ? t[idx] : T(0);
+    }
+}
+
+// U_q = V_q T_q of every block (ld nu, where V_q lies in A): one workgroup
+// per 64 x 64 tile, the k loop up to T's diagonal.
+template <class T>
+__global__ __launch_bounds__(256) void bt_u_kernel(const T* A, const T* Tall, T* U, int64_t su, int nu, int nbb, int B)
+{
+    const int ntc = (nbb + BN - 1) / BN;
+    const int q = blockIdx.y, p = blockIdx.z, ti = blockIdx.x / ntc, tj = blockIdx.x % ntc;
+    const int k = q * nbb, kb = min(nbb, nu - 1 - k), m = nu - k - 1;
+    if (ti * BM >= m || tj * BN >= kb) return;
+    const size_t off = (k + 1) + (size_t)k * nu;
+    GemmShape g{m, kb, min(kb, (tj + 1) * BN), false, false, (int64_t)nu, (int64_t)nbb, (int64_t)nu, 0, 0, 0, 1, 0};
+    gemm_tile<T, GemmBK<T>::value>(g, ti * BM, tj * BN, T(1), A + (size_t)p * nu * nu + off,
+                                   Tall + ((size_t)q * B + p) * nbb * nbb, T(0), U + (size_t)p * su + off);
 }
 
 // ====================================================================== D&C
@@ -1586,7 +1653,7 @@ EigPlan<T>::~EigPlan()
 template <class T>
 static int eig_layout(EigPlan<T>* p, char* base)
 {
-    const size_t B = p->batch, n = p->np, nn = n * n, nb = p->nb, nbb = p->nbb, G = p->G;
+    const size_t B = p->batch, n = p->np, nn = n * n, nb = p->nb, G = p->G;
     size_t off = 0;
     auto take = [&](auto*& ptr, size_t bytes) {
         size_t o = align_up(off);
@@ -1610,7 +1677,6 @@ static int eig_layout(EigPlan<T>* p, char* base)
     for (int** v : {&p->perm, &p->lst, &p->lstD, &p->org, &p->rank, &p->rotp, &p->rotj, &p->kcnt,
                     &p->kpos, &p->kc1, &p->kc2})
         take(*v, B * n * sizeof(int));
-    take(p->Tf, B * 2 * nbb * nbb * sizeof(T));
     take(p->bar, (B * G + 1) * BAR_STRIDE * sizeof(unsigned));
     take(p->err, 64);
     take(p->fro, B * sizeof(T));
@@ -1692,7 +1758,9 @@ static int eig_plan_host(int n, int batch, EigPlan<T>* p, std::vector<std::vecto
 
     // back-transformation block: the rank-nbb updates of Z read and write Z
     // once per block, so the block is as wide as the T factor in LDS allows
-    p->nbb = std::min(bt_max<T>(), n);
+    // (blocks of equal width: their T factors fit the n x n buffer at any order)
+    const int nblk_bt = std::max(1, (p->n - 2) / bt_max<T>() + 1);
+    p->nbb = std::max(1, (p->n - 1 + nblk_bt - 1) / nblk_bt);
     GMC_TRY(eig_layout(p, nullptr));
     return 0;
 }
@@ -1959,66 +2027,65 @@ int syevd_batched(hipStream_t s, EigPlan<T>& p, T* A, T* w)
     // ---------------- back transformation  Z <- H(0)...H(n-2) Z,  Z = Q
     ProfScope ps_bt(s, f64 ? "eig_backtr_f64" : "eig_backtr_f32", 0.0);
     const int nbb = p.nbb;
-    T* Gm = p.Tf;
-    T* Tm = p.Tf + (size_t)B * nbb * nbb;
     if (n > 1) {
-        const size_t lds_t = ((size_t)nbb * (nbb + 1) / 2 + 2 * (size_t)nbb) * sizeof(T);
-        if (!capturing(s))
-            GMC_HIP(hipFuncSetAttribute((const void*)larft_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        (int)lds_t));
         // H(0) ... H(nu-2) of order nu = p.n (a padded reduction's pad rows
         // and reflectors are zero and identities) on the first nu columns of
         // Z (ld n): V has ld nu, Z and the block products ld n
         const int nu = p.n;
         const int64_t nun = (int64_t)nu * nu;
-        const int last = ((nu - 2) / nbb) * nbb;
-        // Every block's T factor depends on its reflectors alone: when the
-        // Gram matrices and factors of all blocks fit in the divide &
-        // conquer's UB (free from here on), they are formed before the loop,
-        // the factors in one launch over (problem, block), instead of one
-        // sequential 16-workgroup launch per block
-        const int nblk = last / nbb + 1;
-        const size_t blk = (size_t)B * nbb * nbb;
-        const bool hoist = 2 * (size_t)nblk * nbb * nbb <= nn;
-        T* Gall = p.UB;
-        T* Tall = p.UB + (size_t)nblk * blk;
-        if (hoist) {
-            for (int k = 0; k <= last; k += nbb) {
-                const int kb = std::min(nbb, nu - 1 - k);
-                const T* V = A + (k + 1) + (size_t)k * nu;
-                GemmShape g1{kb, kb, nu - k - 1, true, false, (int64_t)nu, (int64_t)nu, (int64_t)nbb, nun, nun,
-                             (int64_t)nbb * nbb, B, 0};
-                GMC_TRY(gemm<T>(s, g1, T(1), V, V, T(0), Gall + (size_t)(k / nbb) * blk));
+        const int nblk = nu > 1 ? (nu - 2) / nbb + 1 : 0;
+        GMC_CHECK((size_t)nblk * nbb * nbb <= nn, "syevd: T factors");
+        T* Tall = p.UB;   // the divide & conquer's buffers are free from here on
+        T* U = p.QN;
+        if (nblk > 0) {
+            const size_t lds_t = ((size_t)LT * LT + LT) * sizeof(T);
+            if (!capturing(s))
+                GMC_HIP(hipFuncSetAttribute((const void*)larft_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                            (int)lds_t));
+            const int nt = (nbb + BM - 1) / BM, ntm = (nu - 1 + BM - 1) / BM;
+            hipLaunchKernelGGL(bt_gram_kernel<T>, dim3(nt * (nt + 1) / 2, nblk, B), dim3(256), 0, s, A, Tall, nu, nbb,
+                               B);
+            hipLaunchKernelGGL(larft_kernel<T>, dim3(B, nblk, (nbb + LT - 1) / LT), dim3(256), lds_t, s, Tall, p.tau,
+                               n, nu, nbb);
+            GMC_HIP(hipGetLastError());
+            if (nbb > LT) {
+                // the two triangles of a wider block: T12 = -T1 (G12 T2), every
+                // block the same shape (the last block's columns past kb are
+                // not read by the products below)
+                const int c2 = nbb - LT;
+                GemmShape gw{LT, c2, c2, false, false, (int64_t)nbb, (int64_t)nbb, (int64_t)LT, (int64_t)nbb * nbb,
+                             (int64_t)nbb * nbb, (int64_t)LT * LT, B, 0};
+                for (int q = 0; q < nblk; q++) {
+                    gw.n = gw.k = std::min(nbb, nu - 1 - q * nbb) - LT;
+                    if (gw.n <= 0) continue;
+                    T* Tq = Tall + (size_t)q * B * nbb * nbb;
+                    GMC_TRY(gemm<T>(s, gw, T(1), Tq + (size_t)LT * nbb, Tq + LT + (size_t)LT * nbb, T(0), p.QK));
+                    GemmShape g12{LT, gw.n, LT, false, false, (int64_t)nbb, (int64_t)LT, (int64_t)nbb,
+                                  (int64_t)nbb * nbb, (int64_t)LT * LT, (int64_t)nbb * nbb, B, 0};
+                    GMC_TRY(gemm<T>(s, g12, T(-1), Tq, p.QK, T(0), Tq + (size_t)LT * nbb));
+                }
             }
-            hipLaunchKernelGGL(larft_kernel<T>, dim3(B, nblk), dim3(256), lds_t, s, Gall, p.tau, Tall, n, nu, 0, nbb);
+            hipLaunchKernelGGL(bt_u_kernel<T>, dim3(ntm * nt, nblk, B), dim3(256), 0, s, A, Tall, U, (int64_t)nn, nu,
+                               nbb, B);
             GMC_HIP(hipGetLastError());
         }
-        for (int k = last; k >= 0; k -= nbb) {
-            const int kb = std::min(nbb, nu - 1 - k);
+        for (int q = nblk - 1; q >= 0; q--) {
+            const int k = q * nbb, kb = std::min(nbb, nu - 1 - k);
             const int m = nu - k - 1;
             const T* V = A + (k + 1) + (size_t)k * nu;
             T* Zs = p.Q + (k + 1);
-            if (hoist) {
-                Tm = Tall + (size_t)(k / nbb) * blk;
-            } else {
-                GemmShape g1{kb, kb, m, true, false, (int64_t)nu, (int64_t)nu, (int64_t)nbb, nun, nun,
-                             (int64_t)nbb * nbb, B, 0};
-                GMC_TRY(gemm<T>(s, g1, T(1), V, V, T(0), Gm));
-                hipLaunchKernelGGL(larft_kernel<T>, dim3(B, 1), dim3(256), lds_t, s, Gm, p.tau, Tm, n, nu, k, nbb);
-                GMC_HIP(hipGetLastError());
-            }
             GemmShape g2{kb, nu, m, true, false, (int64_t)nu, (int64_t)n, (int64_t)nbb, nun, (int64_t)nn,
                          (int64_t)nn, B, 0};
-            // own_gemm: the library's MFMA tile (no library workspace)
-            if (p.own_gemm) GMC_TRY(gemm<T>(s, g2, T(1), V, Zs, T(0), p.QK));
-            else GMC_TRY(gemm_big<T>(s, g2, T(1), V, Zs, T(0), p.QK));
-            GemmShape g3{kb, nu, kb, false, false, (int64_t)nbb, (int64_t)nbb, (int64_t)nbb, (int64_t)nbb * nbb,
-                         (int64_t)nn, (int64_t)nn, B, 0};
-            GMC_TRY(gemm<T>(s, g3, T(1), Tm, p.QK, T(0), p.QN));
-            GemmShape g4{m, nu, kb, false, false, (int64_t)nu, (int64_t)nbb, (int64_t)n, nun, (int64_t)nn,
+            GemmShape g4{m, nu, kb, false, false, (int64_t)nu, (int64_t)nbb, (int64_t)n, (int64_t)nn, (int64_t)nn,
                          (int64_t)nn, B, 0};
-            if (p.own_gemm) GMC_TRY(gemm<T>(s, g4, T(-1), V, p.QN, T(1), Zs));
-            else GMC_TRY(gemm_big<T>(s, g4, T(-1), V, p.QN, T(1), Zs));
+            // own_gemm: the library's MFMA tile (no library workspace)
+            if (p.own_gemm) {
+                GMC_TRY(gemm<T>(s, g2, T(1), V, Zs, T(0), p.QK));
+                GMC_TRY(gemm<T>(s, g4, T(-1), U + (k + 1) + (size_t)k * nu, p.QK, T(1), Zs));
+            } else {
+                GMC_TRY(gemm_big<T>(s, g2, T(1), V, Zs, T(0), p.QK));
+                GMC_TRY(gemm_big<T>(s, g4, T(-1), U + (k + 1) + (size_t)k * nu, p.QK, T(1), Zs));
+            }
         }
     }
     if (padded)

@@ -41,7 +41,7 @@ struct EigPlan {
     T *Pu = nullptr, *vg = nullptr;
     T *Q = nullptr, *QK = nullptr, *QN = nullptr, *UB = nullptr;
     T *dsort = nullptr, *zsort = nullptr, *dK = nullptr, *zK = nullptr, *taus = nullptr, *zh = nullptr;
-    T *EV = nullptr, *rotc = nullptr, *rots = nullptr, *Tf = nullptr;
+    T *EV = nullptr, *rotc = nullptr, *rots = nullptr;
     int *perm = nullptr, *lst = nullptr, *lstD = nullptr, *org = nullptr, *rank = nullptr;
     int *rotp = nullptr, *rotj = nullptr, *kcnt = nullptr;
     int *kpos = nullptr, *kc1 = nullptr, *kc2 = nullptr;   // merge GEMM column grouping
