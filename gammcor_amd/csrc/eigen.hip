@@ -955,24 +955,110 @@ __global__ __launch_bounds__(256) void bt_u_kernel(const T* A, const T* Tall, T*
 }
 
 // ====================================================================== D&C
+// The leaves of the divide & conquer: tridiagonal blocks of at most DC_LEAF
+// rows (leaf[l] .. leaf[l + 1] - 1), their ends less the |e| cut off, solved
+// by cyclic Jacobi in LDS, one wave each.  The 8 x 8 pairs of a round's
+// rotations are the wave's 64 lanes (the blocks on or above the diagonal do
+// the work), 15 rounds a sweep, about 6 sweeps: 20 us in one launch where the
+// four levels of merges it replaces took 50 us each.  Eigenvalues ascending
+// into lam, vectors into the leaf's own rows of Q; the rest of Q stays as it
+// is and is not read (a column's rows outside its block count as zero until
+// a merge writes them).
+constexpr int DC_LEAF = 16;
 template <class T>
-__global__ void dc_init_kernel(const T* d, const T* e, const unsigned char* split, T* lam, T* Q, int n)
+__global__ __launch_bounds__(64) void dc_leaf_kernel(const T* d, const T* e, const int* leaf, T* lam, T* Q, int n)
 {
-    const int p = blockIdx.y;
-    const int64_t total = (int64_t)n * n;
-    T* q = Q + (size_t)p * n * n;
-    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-         idx += (int64_t)gridDim.x * blockDim.x) {
-        int r = (int)(idx % n), c = (int)(idx / n);
-        q[idx] = (r == c) ? T(1) : T(0);
-        if (r == 0) {
-            const T* dd = d + (size_t)p * n;
-            const T* ee = e + (size_t)p * n;
-            T v = dd[c];
-            if (c > 0 && split[c - 1]) v -= fabs(ee[c - 1]);
-            if (c < n - 1 && split[c]) v -= fabs(ee[c]);
-            lam[(size_t)p * n + c] = v;
+    __shared__ T A[DC_LEAF][DC_LEAF + 1], V[DC_LEAF][DC_LEAF + 1];
+    const int p = blockIdx.y, s = leaf[blockIdx.x], m = leaf[blockIdx.x + 1] - s, lane = threadIdx.x;
+    const T* dd = d + (size_t)p * n;
+    const T* ee = e + (size_t)p * n;
+    for (int x = lane; x < DC_LEAF * DC_LEAF; x += 64) {
+        const int r = x / DC_LEAF, c = x % DC_LEAF;
+        T v = 0;
+        if (r < m && r == c) {
+            v = dd[s + r];
+            if (r == 0 && s > 0) v -= fabs(ee[s - 1]);
+            if (r == m - 1 && s + m < n) v -= fabs(ee[s + m - 1]);
+        } else if (r < m && c < m && (r == c + 1 || c == r + 1)) {
+            v = ee[s + (r < c ? r : c)];
         }
+        A[r][c] = v;
+        V[r][c] = r == c ? T(1) : T(0);
+    }
+    __syncthreads();
+    T scale = 0;
+    for (int x = lane; x < DC_LEAF * DC_LEAF; x += 64) scale = fmax(scale, fabs(A[x / DC_LEAF][x % DC_LEAF]));
+    scale = wave_max(scale);
+    // the pair t of round r: every two of the 16 rows meet once in 15 rounds
+    auto pair = [](int r, int t, int& x, int& y) {
+        x = t == 0 ? DC_LEAF - 1 : (r + t) % (DC_LEAF - 1);
+        y = t == 0 ? r : (r + DC_LEAF - 1 - t) % (DC_LEAF - 1);
+        if (x > y) {
+            const int z = x;
+            x = y;
+            y = z;
+        }
+    };
+    auto rotation = [&](int x, int y, T& c, T& sn, T& tn) {
+        const T g = A[x][y];
+        c = T(1);
+        sn = tn = T(0);
+        if (g != T(0)) {
+            const T th = (A[y][y] - A[x][x]) / (g + g);
+            tn = copysign(T(1) / (fabs(th) + sqrt(T(1) + th * th)), th);
+            c = T(1) / sqrt(T(1) + tn * tn);
+            sn = tn * c;
+        }
+    };
+    const int i = lane >> 3, k = lane & 7;
+    for (int sweep = 0; sweep < 12; sweep++) {
+        T off = 0;
+        for (int r = 0; r < DC_LEAF - 1; r++) {
+            int pi, qi, pk, qk;
+            pair(r, i, pi, qi);
+            pair(r, k, pk, qk);
+            T ci, si, ti, ck, sk, tk;
+            rotation(pi, qi, ci, si, ti);
+            rotation(pk, qk, ck, sk, tk);
+            const T g = A[pi][qi], app = A[pi][pi], aqq = A[qi][qi];
+            off = fmax(off, fabs(g));
+            const T x00 = A[pi][pk], x01 = A[pi][qk], x10 = A[qi][pk], x11 = A[qi][qk];
+            const T v0 = V[i][pk], v1 = V[i][qk], u0 = V[i + 8][pk], u1 = V[i + 8][qk];
+            __syncthreads();
+            if (i == k) {
+                A[pi][pi] = app - ti * g;
+                A[qi][qi] = aqq + ti * g;
+                A[pi][qi] = A[qi][pi] = T(0);
+            } else if (i < k) {
+                const T y00 = ci * x00 - si * x10, y01 = ci * x01 - si * x11;
+                const T y10 = si * x00 + ci * x10, y11 = si * x01 + ci * x11;
+                const T z00 = ck * y00 - sk * y01, z01 = sk * y00 + ck * y01;
+                const T z10 = ck * y10 - sk * y11, z11 = sk * y10 + ck * y11;
+                A[pi][pk] = A[pk][pi] = z00;
+                A[pi][qk] = A[qk][pi] = z01;
+                A[qi][pk] = A[pk][qi] = z10;
+                A[qi][qk] = A[qk][qi] = z11;
+            }
+            V[i][pk] = ck * v0 - sk * v1;
+            V[i][qk] = sk * v0 + ck * v1;
+            V[i + 8][pk] = ck * u0 - sk * u1;
+            V[i + 8][qk] = sk * u0 + ck * u1;
+            __syncthreads();
+        }
+        // a sweep that met only entries at rounding level has annihilated them
+        if (!(wave_max(off) > Eps<T>::v * scale)) break;
+    }
+    // ascending order (pads beyond m excluded)
+    if (lane < m) {
+        const T w = A[lane][lane];
+        int rank = 0;
+        for (int u = 0; u < m; u++) {
+            const T v = A[u][u];
+            rank += (v < w || (v == w && u < lane)) ? 1 : 0;
+        }
+        lam[(size_t)p * n + s + rank] = w;
+        T* q = Q + (size_t)p * n * n + s + (size_t)(s + rank) * n;
+        for (int r = 0; r < m; r++) q[r] = V[r][lane];
     }
 }
 
@@ -987,6 +1073,7 @@ struct DcBufs {
     T *lam, *Q, *QK, *QN, *UB;
     T *dsort, *zsort, *dK, *zK, *taus, *zh, *EV, *rotc, *rots;
     int *perm, *lst, *lstD, *org, *rank, *rotp, *rotj, *kcnt;
+    int* kneg;   // per merge: deflated columns with a negligible z (the first ones of lstD)
     // Column grouping of the merge product: a non-deflated column t of a
     // merge comes from the first child (rows s..s+m1 only), from both (a
     // deflation rotation mixed one of each) or from the second (rows
@@ -1064,6 +1151,9 @@ __global__ __launch_bounds__(256) void dc_prep_kernel(DcArgs a, DcBufs<T> b)
     const T sgn = beta >= T(0) ? T(1) : T(-1);
     const T rs2 = T(0.70710678118654752440);
     T dmax = 0, zmax = 0;
+    // (non-finite values break the places below; every index stays in range)
+    for (int t = tid; t < m; t += 256) perm[t] = t;
+    __syncthreads();
     for (int t = tid; t < m; t += 256) {
         T D = lam[s + t], z;
         int pos;
@@ -1209,11 +1299,18 @@ __global__ __launch_bounds__(256) void dc_prep_kernel(DcArgs a, DcBufs<T> b)
     }
     if (tid == 0) {
         b.kcnt[po + q] = k;
+        b.kneg[po + q] = m - k0;
         b.kc1[po + q] = n1;
         b.kc2[po + q] = n2;
     }
-    // the rotations on the merge's columns of Q, a row per thread
+    // the rotations on the merge's columns of Q, a row per thread: first the
+    // rows of the columns' other child, zero by meaning, are made so
     for (int r = tid; r < m; r += 256) {
+        for (int t = 0; t < nrot; t++) {
+            const int cx = perm[b.rotp[po + s + t]], cy = perm[b.rotj[po + s + t]];
+            if ((cx < m1) != (r < m1)) Q[(s + r) + (size_t)(s + cx) * n] = T(0);
+            if ((cy < m1) != (r < m1)) Q[(s + r) + (size_t)(s + cy) * n] = T(0);
+        }
         for (int t = 0; t < nrot; t++) {
             const int cx = s + perm[b.rotp[po + s + t]], cy = s + perm[b.rotj[po + s + t]];
             const T c = b.rotc[po + s + t], sn = b.rots[po + s + t];
@@ -1258,7 +1355,10 @@ __global__ __launch_bounds__(256) void dc_secular_kernel(DcArgs a, DcBufs<T> b)
     const int s = a.desc[4 * q];
     const int k = b.kcnt[po + q];
     const int i = x - s;
-    if (i >= k) return;
+    if (i >= k) {
+        if (lane == 0) b.EV[po + x] = b.dsort[po + s + b.lstD[po + s + i - k]];   // a deflated value stays
+        return;
+    }
     const T* dK = b.dK + po + s;
     const T* zK = b.zK + po + s;
     const T beta = b.e[po + s + a.desc[4 * q + 1] - 1];
@@ -1370,10 +1470,13 @@ __global__ __launch_bounds__(256) void dc_secular_kernel(DcArgs a, DcBufs<T> b)
     if (lane == 0) {
         b.org[po + s + i] = o;
         b.taus[po + s + i] = t;
+        b.EV[po + x] = dorg + t;
     }
 }
 
-// Gu-Eisenstat z-hat, one wave per component.
+// The place of every eigenvalue of a merge in ascending order (rank, with the
+// merged eigenvalues into lam) and the Gu-Eisenstat z-hat of the kept
+// components, one wave per column.
 template <class T>
 __global__ __launch_bounds__(256) void dc_zhat_kernel(DcArgs a, DcBufs<T> b)
 {
@@ -1388,6 +1491,21 @@ __global__ __launch_bounds__(256) void dc_zhat_kernel(DcArgs a, DcBufs<T> b)
     const int s = a.desc[4 * q];
     const int k = b.kcnt[po + q];
     const int j = x - s;
+    {
+        const int m = a.desc[4 * q + 1] + a.desc[4 * q + 2];
+        const T* EV = b.EV + po + s;
+        const T v = EV[j];
+        int r = 0;
+        for (int u0 = 0; u0 < m; u0 += 64) {
+            const int u = u0 + lane;
+            const T w = u < m ? EV[u] : T(0);
+            r += __popcll(__ballot(u < m && (w < v || (w == v && u < j))));
+        }
+        if (lane == 0) {
+            b.rank[po + x] = s + r;
+            b.lam[po + s + r] = v;
+        }
+    }
     if (j >= k) return;
     const T* dK = b.dK + po + s;
     const T* taus = b.taus + po + s;
@@ -1407,8 +1525,9 @@ __global__ __launch_bounds__(256) void dc_zhat_kernel(DcArgs a, DcBufs<T> b)
     if (lane == 0) b.zh[po + s + j] = copysign(sqrt(fmax(prod, T(0))), b.zK[po + s + j]);
 }
 
-// Rank-one eigenvectors U (k x k, ld n at column offset s) and gather of the
-// non-deflated columns of Q into QK; one wave per column.
+// Rank-one eigenvectors U (k x k, ld n at column offset s), gather of the
+// kept columns of Q into QK, and the deflated columns of Q to their places
+// in QN; one wave per column.
 template <class T>
 __global__ __launch_bounds__(256) void dc_vec_kernel(DcArgs a, DcBufs<T> b)
 {
@@ -1420,10 +1539,20 @@ __global__ __launch_bounds__(256) void dc_vec_kernel(DcArgs a, DcBufs<T> b)
     const int q = find_merge(a.desc, a.nmerge, x);
     if (q < 0) return;
     const size_t po = (size_t)p * n;
-    const int s = a.desc[4 * q], m = a.desc[4 * q + 1] + a.desc[4 * q + 2];
+    const int s = a.desc[4 * q], m1 = a.desc[4 * q + 1], m = m1 + a.desc[4 * q + 2];
     const int k = b.kcnt[po + q];
     const int i = x - s;
-    if (i >= k) return;
+    if (i >= k) {
+        // a column with a negligible z lives in its child's rows; one that
+        // deflated by a rotation in all of them
+        const int at = b.perm[po + s + b.lstD[po + s + i - k]];
+        const bool full = i - k >= b.kneg[po + q];
+        const int r0 = full || at < m1 ? 0 : m1, r1 = full || at >= m1 ? m : m1;
+        const T* src = b.Q + po * n + s + (size_t)(s + at) * n;
+        T* dst = b.QN + po * n + s + (size_t)b.rank[po + x] * n;
+        for (int r = lane; r < m; r += 64) dst[r] = r >= r0 && r < r1 ? src[r] : T(0);
+        return;
+    }
     const T* dK = b.dK + po + s;
     const T* zh = b.zh + po + s;
     const T dorg = dK[b.org[po + s + i]];
@@ -1433,21 +1562,23 @@ __global__ __launch_bounds__(256) void dc_vec_kernel(DcArgs a, DcBufs<T> b)
         T u = zh[t] / ((dK[t] - dorg) - ti);
         ss += u * u;
     }
-    ss = wave_sum(ss);
+    ss = wave_total(ss);
     const T inv = T(1) / sqrt(ss);
     // U's rows and QK's columns in the grouped order (kpos): their product is
     // the same, and the merge GEMM skips the zero blocks
     const int* kpos = b.kpos + po + s;
     T* U = b.UB + po * n + (size_t)(s + i) * n;
     for (int t = lane; t < k; t += 64) U[kpos[t]] = zh[t] / ((dK[t] - dorg) - ti) * inv;
-    // gather: QK[:, s+kpos[i]] = Q[s.., s + perm[lst[i]]]
-    const int col = s + b.perm[po + s + b.lst[po + s + i]];
-    const T* src = b.Q + po * n + s + (size_t)col * n;
-    T* dst = b.QK + po * n + (size_t)(s + kpos[i]) * n;
-    for (int r = lane; r < m; r += 64) dst[r] = src[r];
+    // gather: QK[:, s+kpos[i]] = Q[s.., s + perm[lst[i]]], the rows the GEMM reads
+    const int at = kpos[i], k1 = b.kc1[po + q], k2 = b.kc2[po + q];
+    const int r0 = at < k1 + k2 ? 0 : m1, r1 = at < k1 ? m1 : m;
+    const T* src = b.Q + po * n + s + (size_t)(s + b.perm[po + s + b.lst[po + s + i]]) * n;
+    T* dst = b.QK + po * n + (size_t)(s + at) * n;
+    for (int r = r0 + lane; r < r1; r += 64) dst[r] = src[r];
 }
 
-// Grouped merge GEMM: QN[:, s..s+k) = QK[:, s..s+k) * U, per merge, as two
+// Grouped merge GEMM: the kept columns of QN = QK[:, s..s+k) * U, written to
+// their sorted places (rank), per merge, as two
 // products that skip QK's zero blocks (columns grouped by kpos): the first
 // child's m1 rows over the first-child and mixed columns, the second child's
 // m2 rows over the mixed and second-child columns.
@@ -1469,7 +1600,7 @@ __global__ __launch_bounds__(256) void dc_gemm_kernel(DcArgs a, DcBufs<T> b, int
     int64_t lt = t - a.desc[4 * q + 3];
     const T* A = b.QK + po * n + (size_t)s * n;
     const T* B = b.UB + po * n + (size_t)s * n;
-    T* C = b.QN + po * n + (size_t)s * n;
+    T* C = b.QN + po * n + s;
     int rows, inner, ti, tj;
     if (lt < (int64_t)nt1 * ntm) {
         // first child's rows over columns [0, k1 + k2)
@@ -1491,69 +1622,7 @@ __global__ __launch_bounds__(256) void dc_gemm_kernel(DcArgs a, DcBufs<T> b, int
     }
     if (tj * 64 >= k || ti * 64 >= rows) return;
     GemmShape g{rows, k, inner, false, false, (int64_t)n, (int64_t)n, (int64_t)n, 0, 0, 0, 1, 0};
-    gemm_tile<T, GemmBK<T>::value>(g, ti * 64, tj * 64, T(1), A, B, T(0), C);
-}
-
-// Eigenvalues of the merged block and the deflated columns appended to QN.
-template <class T>
-__global__ __launch_bounds__(256) void dc_final1_kernel(DcArgs a, DcBufs<T> b)
-{
-    const int n = a.n;
-    const int p = blockIdx.y, x = blockIdx.x;
-    const int q = find_merge(a.desc, a.nmerge, x);
-    if (q < 0) return;
-    const size_t po = (size_t)p * n;
-    const int s = a.desc[4 * q], m = a.desc[4 * q + 1] + a.desc[4 * q + 2];
-    const int k = b.kcnt[po + q];
-    const int t = x - s;
-    if (t < k) {
-        if (threadIdx.x == 0) b.EV[po + x] = b.dK[po + s + b.org[po + s + t]] + b.taus[po + s + t];
-        return;
-    }
-    const int pos = b.lstD[po + s + (t - k)];
-    if (threadIdx.x == 0) b.EV[po + x] = b.dsort[po + s + pos];
-    const int col = s + b.perm[po + s + pos];
-    const T* src = b.Q + po * n + s + (size_t)col * n;
-    T* dst = b.QN + po * n + (size_t)x * n;
-    for (int r = threadIdx.x; r < m; r += 256) dst[r] = src[r];
-}
-
-template <class T>
-__global__ __launch_bounds__(256) void dc_rank_kernel(DcArgs a, DcBufs<T> b)
-{
-    const int n = a.n;
-    const int p = blockIdx.y;
-    const int x = blockIdx.x * 256 + threadIdx.x;
-    if (x >= n) return;
-    const int q = find_merge(a.desc, a.nmerge, x);
-    if (q < 0) return;
-    const size_t po = (size_t)p * n;
-    const int s = a.desc[4 * q], m = a.desc[4 * q + 1] + a.desc[4 * q + 2];
-    const T* EV = b.EV + po + s;
-    const int t = x - s;
-    const T v = EV[t];
-    int r = 0;
-    for (int u = 0; u < m; u++) {
-        T w = EV[u];
-        r += (w < v || (w == v && u < t)) ? 1 : 0;
-    }
-    b.rank[po + x] = s + r;
-}
-
-template <class T>
-__global__ __launch_bounds__(256) void dc_final2_kernel(DcArgs a, DcBufs<T> b)
-{
-    const int n = a.n;
-    const int p = blockIdx.y, x = blockIdx.x;
-    const int q = find_merge(a.desc, a.nmerge, x);
-    if (q < 0) return;
-    const size_t po = (size_t)p * n;
-    const int s = a.desc[4 * q], m = a.desc[4 * q + 1] + a.desc[4 * q + 2];
-    const int dst_col = b.rank[po + x];
-    if (threadIdx.x == 0) b.lam[po + dst_col] = b.EV[po + x];
-    const T* src = b.QN + po * n + (size_t)x * n;
-    T* dst = b.Q + po * n + s + (size_t)dst_col * n;
-    for (int r = threadIdx.x; r < m; r += 256) dst[r] = src[r];
+    gemm_tile<T, GemmBK<T>::value>(g, ti * 64, tj * 64, T(1), A, B, T(0), C, b.rank + po + s);
 }
 
 // Padded problems (EigPlan::np > n): Ap = diag(A, 0) of order np.  The
@@ -1646,7 +1715,7 @@ EigPlan<T>::~EigPlan()
     if (!owns_tables) return;
     for (auto& l : levels)
         if (l.d_desc) (void)hipFree(l.d_desc);
-    if (d_split) (void)hipFree(d_split);
+    if (d_leaf) (void)hipFree(d_leaf);
 }
 
 // Carve the workspace; with base == nullptr only ws_bytes is computed.
@@ -1674,7 +1743,7 @@ static int eig_layout(EigPlan<T>* p, char* base)
     take(p->UB, B * nn * sizeof(T));
     for (T** v : {&p->dsort, &p->zsort, &p->dK, &p->zK, &p->taus, &p->zh, &p->EV, &p->rotc, &p->rots})
         take(*v, B * n * sizeof(T));
-    for (int** v : {&p->perm, &p->lst, &p->lstD, &p->org, &p->rank, &p->rotp, &p->rotj, &p->kcnt,
+    for (int** v : {&p->perm, &p->lst, &p->lstD, &p->org, &p->rank, &p->rotp, &p->rotj, &p->kcnt, &p->kneg,
                     &p->kpos, &p->kc1, &p->kc2})
         take(*v, B * n * sizeof(int));
     take(p->bar, (B * G + 1) * BAR_STRIDE * sizeof(unsigned));
@@ -1690,10 +1759,10 @@ static int eig_layout(EigPlan<T>* p, char* base)
 }
 
 // The plan's host part: G, the divide & conquer levels with their merge
-// descriptors (h_desc, one vector per level) and split flags (h_split).
+// descriptors (h_desc, one vector per level) and leaf boundaries (h_leaf).
 template <class T>
 static int eig_plan_host(int n, int batch, EigPlan<T>* p, std::vector<std::vector<int>>& h_desc,
-                         std::vector<unsigned char>& h_split)
+                         std::vector<int>& h_leaf)
 {
     GMC_CHECK(n >= 1 && batch >= 1, "eig_plan: bad sizes n=%d batch=%d", n, batch);
     p->n = n;
@@ -1717,44 +1786,37 @@ static int eig_plan_host(int n, int batch, EigPlan<T>* p, std::vector<std::vecto
     p->G = std::max(1, std::min(nblk, ncu / batch));
     GMC_CHECK(batch <= ncu, "eig_plan: batch %d exceeds the %d co-resident problems", batch, ncu);
 
-    // divide & conquer tree: recursive halving down to single rows
-    struct Node { int s, m1, m2, h; };
-    std::vector<Node> nodes;
-    std::vector<unsigned char> split(n > 1 ? n - 1 : 1, 0);
-    std::function<int(int, int)> build = [&](int s, int m) -> int {
-        if (m == 1) return 0;
-        int m1 = m / 2;
-        split[s + m1 - 1] = 1;
-        int h = 1 + std::max(build(s, m1), build(s + m1, m - m1));
-        nodes.push_back({s, m1, m - m1, h});
-        return h;
-    };
-    int H = build(0, n);
-    p->levels.assign(H, DcLevel{});
-    for (int h = 1; h <= H; h++) {
-        std::vector<Node> lv;
-        for (auto& nd : nodes)
-            if (nd.h == h) lv.push_back(nd);
-        std::sort(lv.begin(), lv.end(), [](const Node& x, const Node& y) { return x.s < y.s; });
-        std::vector<int> desc;
+    // divide & conquer tree: halved to the same depth everywhere, until no
+    // leaf has more than DC_LEAF rows (sizes of one depth differ by at most
+    // one, so every row takes part in one merge per level)
+    int depth = 0;
+    while (((n - 1) >> depth) + 1 > DC_LEAF) depth++;
+    std::vector<int> cut{0, n};
+    p->levels.assign(depth, DcLevel{});
+    h_desc.assign(depth, {});
+    for (int lev = depth; lev >= 1; lev--) {
+        std::vector<int> next, &desc = h_desc[lev - 1];
         int64_t off = 0;
         int maxm = 0;
-        for (auto& nd : lv) {
-            int m = nd.m1 + nd.m2;
-            desc.insert(desc.end(), {nd.s, nd.m1, nd.m2, (int)off});
+        for (size_t i = 0; i + 1 < cut.size(); i++) {
+            const int s0 = cut[i], m = cut[i + 1] - s0, m1 = m / 2, m2 = m - m1;
+            desc.insert(desc.end(), {s0, m1, m2, (int)off});
             // the merge product's tiles: rows of each child's part times the columns
-            int64_t tm = (m + 63) / 64;
-            off += ((nd.m1 + 63) / 64 + (nd.m2 + 63) / 64) * tm;
+            off += (int64_t)((m1 + 63) / 64 + (m2 + 63) / 64) * ((m + 63) / 64);
             maxm = std::max(maxm, m);
+            next.push_back(s0);
+            next.push_back(s0 + m1);
         }
+        next.push_back(n);
         GMC_CHECK(off < (1LL << 31), "eig_plan: tile count overflow");
-        DcLevel& L = p->levels[h - 1];
-        L.nmerge = (int)lv.size();
+        DcLevel& L = p->levels[lev - 1];
+        L.nmerge = (int)cut.size() - 1;
         L.tiles = off;
         L.maxm = maxm;
-        h_desc.push_back(std::move(desc));
+        cut = std::move(next);
     }
-    h_split = std::move(split);
+    p->nleaf = (int)cut.size() - 1;
+    h_leaf = std::move(cut);
 
     // back-transformation block: the rank-nbb updates of Z read and write Z
     // once per block, so the block is as wide as the T factor in LDS allows
@@ -1771,8 +1833,8 @@ size_t eig_workspace_bytes(int n, int batch)
     EigPlan<T> p;
     p.owns_tables = false;
     std::vector<std::vector<int>> h_desc;
-    std::vector<unsigned char> h_split;
-    if (eig_plan_host(n, batch, &p, h_desc, h_split) != 0) return SIZE_MAX;
+    std::vector<int> h_leaf;
+    if (eig_plan_host(n, batch, &p, h_desc, h_leaf) != 0) return SIZE_MAX;
     return p.ws_bytes;
 }
 template size_t eig_workspace_bytes<double>(int, int);
@@ -1782,16 +1844,16 @@ template <class T>
 int eig_plan(int n, int batch, EigPlan<T>* p)
 {
     std::vector<std::vector<int>> h_desc;
-    std::vector<unsigned char> h_split;
-    GMC_TRY(eig_plan_host(n, batch, p, h_desc, h_split));
+    std::vector<int> h_leaf;
+    GMC_TRY(eig_plan_host(n, batch, p, h_desc, h_leaf));
     p->owns_tables = true;
     for (size_t h = 0; h < h_desc.size(); h++) {
         DcLevel& L = p->levels[h];
         GMC_HIP(hipMalloc(&L.d_desc, h_desc[h].size() * sizeof(int)));
         GMC_HIP(hipMemcpy(L.d_desc, h_desc[h].data(), h_desc[h].size() * sizeof(int), hipMemcpyHostToDevice));
     }
-    GMC_HIP(hipMalloc(&p->d_split, h_split.size()));
-    GMC_HIP(hipMemcpy(p->d_split, h_split.data(), h_split.size(), hipMemcpyHostToDevice));
+    GMC_HIP(hipMalloc(&p->d_leaf, h_leaf.size() * sizeof(int)));
+    GMC_HIP(hipMemcpy(p->d_leaf, h_leaf.data(), h_leaf.size() * sizeof(int), hipMemcpyHostToDevice));
     return 0;
 }
 
@@ -1799,13 +1861,13 @@ template <class T>
 int eig_plan_at(int n, int batch, EigPlan<T>* p, void* mem, size_t mem_bytes, size_t* used, hipStream_t s)
 {
     std::vector<std::vector<int>> h_desc;
-    std::vector<unsigned char> h_split;
-    GMC_TRY(eig_plan_host(n, batch, p, h_desc, h_split));
+    std::vector<int> h_leaf;
+    GMC_TRY(eig_plan_host(n, batch, p, h_desc, h_leaf));
     p->owns_tables = false;
     // the tables, then the workspace (bound by the caller at mem + *used)
     size_t need = 0;
     for (auto& d : h_desc) need = align_up(need) + d.size() * sizeof(int);
-    need = align_up(align_up(need) + h_split.size()) + p->ws_bytes;
+    need = align_up(align_up(need) + h_leaf.size() * sizeof(int)) + p->ws_bytes;
     GMC_CHECK(need <= mem_bytes, "syevd: n=%d, batch=%d needs %zu bytes of device scratch, more than the %zu "
               "available", n, batch, need, mem_bytes);
     char* base = static_cast<char*>(mem);
@@ -1818,9 +1880,9 @@ int eig_plan_at(int n, int batch, EigPlan<T>* p, void* mem, size_t mem_bytes, si
         off += bytes;
     }
     off = align_up(off);
-    p->d_split = reinterpret_cast<unsigned char*>(base + off);
-    GMC_HIP(hipMemcpyAsync(base + off, h_split.data(), h_split.size(), hipMemcpyHostToDevice, s));
-    off += h_split.size();
+    p->d_leaf = reinterpret_cast<int*>(base + off);
+    GMC_HIP(hipMemcpyAsync(base + off, h_leaf.data(), h_leaf.size() * sizeof(int), hipMemcpyHostToDevice, s));
+    off += h_leaf.size() * sizeof(int);
     // the host vectors go out of scope: the copies must have left them
     GMC_HIP(hipStreamSynchronize(s));
     *used = align_up(off);
@@ -2003,8 +2065,8 @@ int syevd_batched(hipStream_t s, EigPlan<T>& p, T* A, T* w)
 
     // ---------------- divide & conquer
     DcBufs<T> b{p.e, w, p.Q, p.QK, p.QN, p.UB, p.dsort, p.zsort, p.dK, p.zK, p.taus, p.zh, p.EV, p.rotc, p.rots,
-                p.perm, p.lst, p.lstD, p.org, p.rank, p.rotp, p.rotj, p.kcnt, p.kpos, p.kc1, p.kc2};
-    hipLaunchKernelGGL(dc_init_kernel<T>, dim3(grid1(nn), B), dim3(256), 0, s, p.d, p.e, p.d_split, w, p.Q, n);
+                p.perm, p.lst, p.lstD, p.org, p.rank, p.rotp, p.rotj, p.kcnt, p.kneg, p.kpos, p.kc1, p.kc2};
+    hipLaunchKernelGGL(dc_leaf_kernel<T>, dim3(p.nleaf, B), dim3(64), 0, s, p.d, p.e, p.d_leaf, w, b.Q, n);
     GMC_HIP(hipGetLastError());
     for (auto& L : p.levels) {
         DcArgs a{n, L.nmerge, B, L.d_desc};
@@ -2017,14 +2079,13 @@ int syevd_batched(hipStream_t s, EigPlan<T>& p, T* A, T* w)
             ProfScope ps(s, sizeof(T) == 8 ? "dc_merge_gemm_f64" : "dc_merge_gemm_f32", 0.0);
             hipLaunchKernelGGL(dc_gemm_kernel<T>, dim3((unsigned)(B * L.tiles)), dim3(256), 0, s, a, b, L.tiles);
         }
-        hipLaunchKernelGGL(dc_final1_kernel<T>, dim3(n, B), dim3(256), 0, s, a, b);
-        hipLaunchKernelGGL(dc_rank_kernel<T>, dim3((n + 255) / 256, B), dim3(256), 0, s, a, b);
-        hipLaunchKernelGGL(dc_final2_kernel<T>, dim3(n, B), dim3(256), 0, s, a, b);
         GMC_HIP(hipGetLastError());
+        std::swap(b.Q, b.QN);   // the merged vectors are the next level's
     }
+    T* const Z = b.Q;
 
     ps_dc.close();
-    // ---------------- back transformation  Z <- H(0)...H(n-2) Z,  Z = Q
+    // ---------------- back transformation  Z <- H(0)...H(n-2) Z
     ProfScope ps_bt(s, f64 ? "eig_backtr_f64" : "eig_backtr_f32", 0.0);
     const int nbb = p.nbb;
     if (n > 1) {
@@ -2036,7 +2097,7 @@ int syevd_batched(hipStream_t s, EigPlan<T>& p, T* A, T* w)
         const int nblk = nu > 1 ? (nu - 2) / nbb + 1 : 0;
         GMC_CHECK((size_t)nblk * nbb * nbb <= nn, "syevd: T factors");
         T* Tall = p.UB;   // the divide & conquer's buffers are free from here on
-        T* U = p.QN;
+        T* U = b.QN;
         if (nblk > 0) {
             const size_t lds_t = ((size_t)LT * LT + LT) * sizeof(T);
             if (!capturing(s))
@@ -2073,7 +2134,7 @@ int syevd_batched(hipStream_t s, EigPlan<T>& p, T* A, T* w)
             const int k = q * nbb, kb = std::min(nbb, nu - 1 - k);
             const int m = nu - k - 1;
             const T* V = A + (k + 1) + (size_t)k * nu;
-            T* Zs = p.Q + (k + 1);
+            T* Zs = Z + (k + 1);
             GemmShape g2{kb, nu, m, true, false, (int64_t)nu, (int64_t)n, (int64_t)nbb, nun, (int64_t)nn,
                          (int64_t)nn, B, 0};
             GemmShape g4{m, nu, kb, false, false, (int64_t)nu, (int64_t)nbb, (int64_t)n, (int64_t)nn, (int64_t)nn,
@@ -2089,10 +2150,10 @@ int syevd_batched(hipStream_t s, EigPlan<T>& p, T* A, T* w)
         }
     }
     if (padded)
-        hipLaunchKernelGGL(pad_out_kernel<T>, dim3(grid1((int64_t)p.n * p.n), B), dim3(256), 0, s, p.Q, p.wp, n, Au,
+        hipLaunchKernelGGL(pad_out_kernel<T>, dim3(grid1((int64_t)p.n * p.n), B), dim3(256), 0, s, Z, p.wp, n, Au,
                            wu, p.n);
     else
-        hipLaunchKernelGGL(copy_kernel<T>, dim3(grid1((int64_t)B * nn)), dim3(256), 0, s, p.Q, A, (int64_t)B * nn);
+        hipLaunchKernelGGL(copy_kernel<T>, dim3(grid1((int64_t)B * nn)), dim3(256), 0, s, Z, A, (int64_t)B * nn);
     GMC_HIP(hipGetLastError());
     return 0;
 }

@@ -34,7 +34,8 @@ struct EigPlan {
     int ncu = 0;            // compute units of the device
     int mres = 0;           // largest trailing order the resident reduction takes (sytrd_resident.hpp)
     std::vector<DcLevel> levels;
-    unsigned char* d_split = nullptr;   // split flags (n)
+    int nleaf = 0;
+    int* d_leaf = nullptr;              // first row of every leaf, then n
     size_t ws_bytes = 0;
     // carved device scratch
     T *W = nullptr, *X = nullptr, *d = nullptr, *e = nullptr, *tau = nullptr, *part = nullptr;
@@ -43,7 +44,7 @@ struct EigPlan {
     T *dsort = nullptr, *zsort = nullptr, *dK = nullptr, *zK = nullptr, *taus = nullptr, *zh = nullptr;
     T *EV = nullptr, *rotc = nullptr, *rots = nullptr;
     int *perm = nullptr, *lst = nullptr, *lstD = nullptr, *org = nullptr, *rank = nullptr;
-    int *rotp = nullptr, *rotj = nullptr, *kcnt = nullptr;
+    int *rotp = nullptr, *rotj = nullptr, *kcnt = nullptr, *kneg = nullptr;
     int *kpos = nullptr, *kc1 = nullptr, *kc2 = nullptr;   // merge GEMM column grouping
     unsigned* bar = nullptr;
     int* err = nullptr;
@@ -53,7 +54,7 @@ struct EigPlan {
     // bind clears it, later ones add to it (eig_check_error reads and clears)
     bool clear_err = true;
     bool bound = false;
-    bool owns_tables = true;   // d_desc / d_split allocated by eig_plan (else placed by eig_plan_at)
+    bool owns_tables = true;   // d_desc / d_leaf allocated by eig_plan (else placed by eig_plan_at)
     bool own_gemm = false;     // back-transformation products on the library's MFMA tile only
     EigPlan() = default;
     EigPlan(const EigPlan&) = delete;

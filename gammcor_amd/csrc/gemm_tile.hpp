@@ -42,9 +42,11 @@ template <> struct Mfma<float> {
 constexpr int BM = 64, BN = 64;
 
 // One 64x64 tile (rows bi.., cols bj..) of C = alpha op(A) op(B) + beta C.
-// Must be called by all 256 threads of the workgroup.
+// Must be called by all 256 threads of the workgroup.  With cmap (beta == 0)
+// column j of the result is stored as column cmap[j] of C.
 template <class T, int BK>
-__device__ void gemm_tile(const GemmShape& g, int bi, int bj, T alpha, const T* A, const T* B, T beta, T* C)
+__device__ void gemm_tile(const GemmShape& g, int bi, int bj, T alpha, const T* A, const T* B, T beta, T* C,
+                          const int* cmap = nullptr)
 {
     __shared__ T As[BK][BM + 1];
     __shared__ T Bs[BK][BN + 1];
@@ -138,7 +140,7 @@ __device__ void gemm_tile(const GemmShape& g, int bi, int bj, T alpha, const T* 
                 if (i < g.m && j < g.n && (g.uplo == 0 || i >= j)) {
                     T v = alpha * acc[x][y][r];
                     if (beta != T(0)) v += beta * cpre[x][y][r];
-                    C[i + (int64_t)j * g.ldc] = v;
+                    C[i + (int64_t)(cmap ? cmap[j] : j) * g.ldc] = v;
                 }
             }
 }
