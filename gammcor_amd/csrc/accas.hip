@@ -19,6 +19,7 @@
 #include "oa_policy.hpp"
 #include "gemm.hpp"
 #include "prof.hpp"
+#include "wave_ops.hpp"
 
 namespace gmc {
 
@@ -578,8 +579,15 @@ int integrand_weights(hipStream_t st, const AcSystem& a, const double* cicoef, d
 // A(0) and A(1) combined affinely (A+-B is affine in alpha; ERPASYMM1
 // symmetrises, interpa.f:1680-1687).  One workgroup per 64 x 64 tile on or
 // below the diagonal: each base tile and its transposed partner are read
-// once and symmetrised in LDS, then every alpha point's tile and its mirror
-// are written along columns.
+// once and symmetrised in LDS, then the alpha points' tiles and their mirrors
+// are written along columns.  blockIdx.z: A+ or A-; blockIdx.y: a share of
+// the alpha points where the tiles alone would leave the chip idle (order
+// 410, 8 points: 28 workgroups took 85 us, 448 take 11).
+inline dim3 form_grid(int ntile, int nsys, int nalpha)
+{
+    const int share = std::max(1, std::min(nalpha, 1024 / std::max(1, 2 * ntile * nsys)));
+    return dim3(ntile, share * nsys, 2);
+}
 template <class T>
 __global__ __launch_bounds__(256) void form_kernel(const double* p0, const double* p1, const double* m0,
                                                    const double* m1, const double* alphas, int nalpha, T* Ap, T* Am,
@@ -601,11 +609,12 @@ __global__ __launch_bounds__(256) void form_kernel(const double* p0, const doubl
         for (int y = ty; y < 64; y += 4) dst[y][tx] = 0.5 * (dst[y][tx] + tmp[tx][y]);
         __syncthreads();
     };
-    for (int which = 0; which < 2; which++) {
+    {
+        const int which = blockIdx.z;
         load_sym(which ? m0 : p0, s0);
         load_sym(which ? m1 : p1, s1);
         T* out = which ? Am : Ap;
-        for (int b = 0; b < nalpha; b++) {
+        for (int b = blockIdx.y; b < nalpha; b += gridDim.y) {
             const double al = alphas[b];
             T* o = out + (size_t)b * n * n;
             for (int y = ty; y < 64; y += 4) {
@@ -628,16 +637,17 @@ __global__ __launch_bounds__(256) void form_kernel(const double* p0, const doubl
 // tolerance (8 eps max(|d|, |z|) of a merge) as it is without them - a pad
 // above the spectrum would raise it; S, M and Y are zero on them, and the
 // integrand reads only the system's own block.  One workgroup per 64 x 64
-// tile on or below the diagonal and system (blockIdx.y), writing the tile of
-// every alpha point.
+// tile on or below the diagonal, system and share of its alpha points
+// (blockIdx.y; form_grid).
 template <class T>
-__global__ __launch_bounds__(256) void form_pad_kernel(const BatchSys* sys, const double* alphas, int nalpha,
-                                                       T* Ap, T* Am, int npad)
+__global__ __launch_bounds__(256) void form_pad_kernel(const BatchSys* sys, int nsys, const double* alphas,
+                                                       int nalpha, T* Ap, T* Am, int npad)
 {
     __shared__ double s0[64][65], s1[64][65], tmp[64][65];
     int ti, tj;
     lower_tile(blockIdx.x, ti, tj);
-    const BatchSys sy = sys[blockIdx.y];
+    const int nshare = gridDim.y / nsys, ksys = blockIdx.y / nshare;
+    const BatchSys sy = sys[ksys];
     const int n = sy.n;
     const int i0 = ti * 64, j0 = tj * 64, tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
     auto load_sym = [&](const double* X, double (*dst)[65]) {
@@ -651,13 +661,14 @@ __global__ __launch_bounds__(256) void form_pad_kernel(const BatchSys* sys, cons
         for (int y = ty; y < 64; y += 4) dst[y][tx] = 0.5 * (dst[y][tx] + tmp[tx][y]);
         __syncthreads();
     };
-    for (int which = 0; which < 2; which++) {
+    {
+        const int which = blockIdx.z;
         load_sym(which ? sy.m0 : sy.p0, s0);
         load_sym(which ? sy.m1 : sy.p1, s1);
         T* out = which ? Am : Ap;
-        for (int a = 0; a < nalpha; a++) {
+        for (int a = blockIdx.y % nshare; a < nalpha; a += nshare) {
             const double al = alphas[a];
-            T* o = out + ((size_t)blockIdx.y * nalpha + a) * npad * npad;
+            T* o = out + ((size_t)ksys * nalpha + a) * npad * npad;
             for (int y = ty; y < 64; y += 4) {
                 const int i = i0 + tx, j = j0 + y;
                 if (i < npad && j < npad) {
@@ -700,14 +711,21 @@ __global__ __launch_bounds__(256) void dot_batch_kernel(const BatchSys* sys, int
     if (threadIdx.x == 0) partial[(size_t)b * gridDim.x + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
-__global__ void sum_partials_batch_kernel(const double* partial, int np, const BatchSys* sys, int nalpha, double* W,
-                                          int nb)
+// The sum of np values by one wave, in a fixed order (every lane gets it).
+__device__ inline double partials_total(const double* x, int np)
 {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nb) return;
     double s = 0.0;
-    for (int i = 0; i < np; i++) s += partial[(size_t)b * np + i];
-    W[b] = s + sys[b / nalpha].wdiag;
+    for (int i = threadIdx.x; i < np; i += 64) s += x[i];
+    return wave_total(s);
+}
+
+// One wave per problem.
+__global__ __launch_bounds__(64) void sum_partials_batch_kernel(const double* partial, int np, const BatchSys* sys,
+                                                                int nalpha, double* W)
+{
+    const int b = blockIdx.x;
+    const double s = partials_total(partial + (size_t)b * np, np);
+    if (threadIdx.x == 0) W[b] = s + sys[b / nalpha].wdiag;
 }
 
 // x[0..n) = 0 (a kernel, not a memset: the solve sequence may be captured)
@@ -796,13 +814,12 @@ __global__ __launch_bounds__(256) void dot_lower_kernel(const double* Gw, const 
     if (threadIdx.x == 0) partial[(size_t)b * gridDim.x + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
-__global__ void sum_partials_kernel(const double* partial, int np, const double* wdiag, double* W, int nb)
+// (one thread per problem took 82 us for its 1024 partials; a wave 5)
+__global__ __launch_bounds__(64) void sum_partials_kernel(const double* partial, int np, const double* wdiag, double* W)
 {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nb) return;
-    double s = 0.0;
-    for (int i = 0; i < np; i++) s += partial[(size_t)b * np + i];
-    W[b] = s + *wdiag;
+    const int b = blockIdx.x;
+    const double s = partials_total(partial + (size_t)b * np, np);
+    if (threadIdx.x == 0) W[b] = s + *wdiag;
 }
 
 template <class T>
@@ -846,11 +863,11 @@ int erpa_batched(hipStream_t st, ErpaPlan<T>& p, const AbPair& ab, const double*
     const int nt64f = (n + 63) / 64;
     if (bt) {
         // the batching form: alphas are already on the device
-        hipLaunchKernelGGL(form_pad_kernel<T>, dim3(nt64f * (nt64f + 1) / 2, bt->nsys), blk, 0, st, bt->sys, alphas,
-                           nalpha, E, Tb, n);
+        hipLaunchKernelGGL(form_pad_kernel<T>, form_grid(nt64f * (nt64f + 1) / 2, bt->nsys, nalpha), blk, 0, st, bt->sys,
+                           bt->nsys, alphas, nalpha, E, Tb, n);
     } else {
         GMC_HIP(hipMemcpyAsync(d_al, alphas, nalpha * sizeof(double), hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(form_kernel<T>, dim3(nt64f * (nt64f + 1) / 2), blk, 0, st, ab.p0, ab.p1, ab.m0, ab.m1,
+        hipLaunchKernelGGL(form_kernel<T>, form_grid(nt64f * (nt64f + 1) / 2, 1, B), blk, 0, st, ab.p0, ab.p1, ab.m0, ab.m1,
                            d_al, B, E, Tb, n);
     }
     GMC_HIP(hipGetLastError());
@@ -894,11 +911,11 @@ int erpa_batched(hipStream_t st, ErpaPlan<T>& p, const AbPair& ab, const double*
         GMC_TRY(gemm_big<T>(st, gP, T(1), E, E, T(0), Sb));
         if (bt) {
             hipLaunchKernelGGL(dot_batch_kernel<T>, dim3(npart, Bp), blk, 0, st, bt->sys, nalpha, Sb, n, partial);
-            hipLaunchKernelGGL(sum_partials_batch_kernel, dim3((Bp + 63) / 64), dim3(64), 0, st, partial, npart,
-                               bt->sys, nalpha, out.W, Bp);
+            hipLaunchKernelGGL(sum_partials_batch_kernel, dim3(Bp), dim3(64), 0, st, partial, npart,
+                               bt->sys, nalpha, out.W);
         } else {
             hipLaunchKernelGGL(dot_lower_kernel<T>, dim3(npart, B), blk, 0, st, Gw, Sb, n, partial);
-            hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(64), 0, st, partial, npart, wdiag, out.W, B);
+            hipLaunchKernelGGL(sum_partials_kernel, dim3(B), dim3(64), 0, st, partial, npart, wdiag, out.W);
         }
         GMC_HIP(hipGetLastError());
     }
@@ -2087,12 +2104,12 @@ int erpa_batched_mixed(hipStream_t st, EigPlan<float>& ep, int n, const AbPair& 
     const int nt64f = (n + 63) / 64;
     if (bt) {
         // the batching form: alphas are already on the device
-        hipLaunchKernelGGL(form_pad_kernel<double>, dim3(nt64f * (nt64f + 1) / 2, bt->nsys), blk, 0, st, bt->sys,
-                           alphas, nalpha, Ap, Am, n);
+        hipLaunchKernelGGL(form_pad_kernel<double>, form_grid(nt64f * (nt64f + 1) / 2, bt->nsys, nalpha), blk, 0, st,
+                           bt->sys, bt->nsys, alphas, nalpha, Ap, Am, n);
         hipLaunchKernelGGL(pad_diag_set_kernel, dim3(B), blk, 0, st, bt->sys, nalpha, Ap, n, 1.0);
     } else {
         GMC_HIP(hipMemcpyAsync(d_al, alphas, nalpha * sizeof(double), hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(form_kernel<double>, dim3(nt64f * (nt64f + 1) / 2), blk, 0, st, ab.p0, ab.p1, ab.m0,
+        hipLaunchKernelGGL(form_kernel<double>, form_grid(nt64f * (nt64f + 1) / 2, 1, B), blk, 0, st, ab.p0, ab.p1, ab.m0,
                            ab.m1, d_al, B, Ap, Am, n);
     }
     // eig(A+) in FP32, refined in FP64
@@ -2250,11 +2267,11 @@ int erpa_batched_mixed(hipStream_t st, EigPlan<float>& ep, int n, const AbPair& 
     GMC_TRY(gemm_big<double>(st, gP, 1.0, Gb, Gb, 0.0, Am));
     if (bt) {
         hipLaunchKernelGGL(dot_batch_kernel<double>, dim3(npart, B), blk, 0, st, bt->sys, nalpha, Am, n, partial);
-        hipLaunchKernelGGL(sum_partials_batch_kernel, dim3((B + 63) / 64), dim3(64), 0, st, partial, npart, bt->sys,
-                           nalpha, out.W, B);
+        hipLaunchKernelGGL(sum_partials_batch_kernel, dim3(B), dim3(64), 0, st, partial, npart, bt->sys,
+                           nalpha, out.W);
     } else {
         hipLaunchKernelGGL(dot_lower_kernel<double>, dim3(npart, B), blk, 0, st, Gw, Am, n, partial);
-        hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(64), 0, st, partial, npart, wdiag, out.W, B);
+        hipLaunchKernelGGL(sum_partials_kernel, dim3(B), dim3(64), 0, st, partial, npart, wdiag, out.W);
     }
     GMC_HIP(hipGetLastError());
     return 0;
@@ -2295,7 +2312,7 @@ int integrand_from_y(hipStream_t st, int n, const double* Y, const double* eig, 
     GemmShape gP{n, n, n, false, true, n, n, n, 0, 0, 0, 1, 1};
     GMC_TRY(gemm_big<double>(st, gP, 1.0, Yf, Yf, 0.0, P));
     hipLaunchKernelGGL(dot_lower_kernel<double>, dim3(npart, 1), dim3(256), 0, st, Gw, P, n, partial);
-    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(64), 0, st, partial, npart, wdiag, W, 1);
+    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(64), 0, st, partial, npart, wdiag, W);
     GMC_HIP(hipGetLastError());
     return 0;
 }

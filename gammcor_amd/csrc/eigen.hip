@@ -902,33 +902,40 @@ __global__ __launch_bounds__(256) void larft_kernel(T* G, const T* tau, int n, i
     for (int h = LT_BASE; h < LT && h < kb; h *= 2) {
         // pairs of triangles T1 at d, T2 at d + h: W = U12 T2 into the unused
         // block below the diagonal, then T12 = -T1 W
-        const int nout = LT / 2 * h;   // outputs over all pairs
+        // (4 x 4 outputs per thread)
+        const int ntile = LT / 2 * h / 16, hq = h / 4;
         for (int pass = 0; pass < 2; pass++) {
-            for (int idx = tid; idx < nout / 4; idx += 256) {
-                const int e = idx * 4, d = e / (h * h) * 2 * h, x = e % (h * h), r = x % h, c = x / h;
-                T acc[4] = {T(0), T(0), T(0), T(0)};
-                if (pass == 0) {
-                    // W(r, c) = sum_{l <= c} U12(r, l) T2(l, c)
-                    for (int l = 0; l <= c; l++) {
-                        const T y = t[d + h + l + (d + h + c) * LT];
-                        const T* u = t + d + r + (d + h + l) * LT;
+            for (int idx = tid; idx < ntile; idx += 256) {
+                const int d = idx / (hq * hq) * 2 * h, x = idx % (hq * hq), r = x % hq * 4, c = x / hq * 4;
+                T acc[4][4];
 #pragma unroll
-                        for (int z = 0; z < 4; z++) acc[z] += u[z] * y;
-                    }
-                } else {
-                    // T12(r, c) = -sum_{l >= r} T1(r, l) W(l, c)
-                    for (int l = r; l < h; l++) {
-                        const T y = t[d + h + l + (d + c) * LT];
-                        const T* u = t + d + r + (d + l) * LT;
+                for (int y = 0; y < 4; y++)
 #pragma unroll
-                        for (int z = 0; z < 4; z++) acc[z] += (l >= r + z ? u[z] : T(0)) * y;
+                    for (int z = 0; z < 4; z++) acc[y][z] = T(0);
+                // pass 0: W(r, c) = sum_{l <= c} U12(r, l) T2(l, c); pass 1:
+                // T12(r, c) = -sum_{l >= r} T1(r, l) W(l, c)
+                const int l0 = pass == 0 ? 0 : r, l1 = pass == 0 ? c + 4 : h;
+                const T* u = t + d + r + (pass == 0 ? d + h : d) * LT;
+                const T* w = t + d + h + (pass == 0 ? d + h + c : d + c) * LT;
+                for (int l = l0; l < l1; l++) {
+                    T uu[4], ww[4];
+#pragma unroll
+                    for (int z = 0; z < 4; z++) {
+                        uu[z] = pass == 0 || l >= r + z ? u[z + l * LT] : T(0);
+                        ww[z] = pass == 1 || l <= c + z ? w[l + z * LT] : T(0);
                     }
+#pragma unroll
+                    for (int y = 0; y < 4; y++)
+#pragma unroll
+                        for (int z = 0; z < 4; z++) acc[y][z] += uu[z] * ww[y];
                 }
 #pragma unroll
-                for (int z = 0; z < 4; z++) {
-                    if (pass == 0) t[d + h + r + z + (d + c) * LT] = acc[z];
-                    else t[d + r + z + (d + h + c) * LT] = -acc[z];
-                }
+                for (int y = 0; y < 4; y++)
+#pragma unroll
+                    for (int z = 0; z < 4; z++) {
+                        if (pass == 0) t[d + h + r + z + (d + c + y) * LT] = acc[y][z];
+                        else t[d + r + z + (d + h + c + y) * LT] = -acc[y][z];
+                    }
             }
             __syncthreads();
         }
@@ -986,28 +993,36 @@ __global__ __launch_bounds__(64) void dc_leaf_kernel(const T* d, const T* e, con
         V[r][c] = r == c ? T(1) : T(0);
     }
     __syncthreads();
-    T scale = 0;
-    for (int x = lane; x < DC_LEAF * DC_LEAF; x += 64) scale = fmax(scale, fabs(A[x / DC_LEAF][x % DC_LEAF]));
-    scale = wave_max(scale);
+    // entries scaled by a power of two to at most 1 (the rotations square them)
+    T big = 0;
+    for (int x = lane; x < DC_LEAF * DC_LEAF; x += 64) big = fmax(big, fabs(A[x / DC_LEAF][x % DC_LEAF]));
+    big = wave_max(big);
+    int ex = 0;
+    if (big > T(0) && big < T(INFINITY)) frexp(big, &ex);
+    __syncthreads();
+    for (int x = lane; x < DC_LEAF * DC_LEAF; x += 64) A[x / DC_LEAF][x % DC_LEAF] = ldexp(A[x / DC_LEAF][x % DC_LEAF], -ex);
+    __syncthreads();
     // the pair t of round r: every two of the 16 rows meet once in 15 rounds
     auto pair = [](int r, int t, int& x, int& y) {
-        x = t == 0 ? DC_LEAF - 1 : (r + t) % (DC_LEAF - 1);
-        y = t == 0 ? r : (r + DC_LEAF - 1 - t) % (DC_LEAF - 1);
-        if (x > y) {
-            const int z = x;
-            x = y;
-            y = z;
-        }
+        int a = r + t, c = r + DC_LEAF - 1 - t;
+        a = t == 0 ? DC_LEAF - 1 : (a >= DC_LEAF - 1 ? a - (DC_LEAF - 1) : a);
+        c = t == 0 ? r : (c >= DC_LEAF - 1 ? c - (DC_LEAF - 1) : c);
+        x = a < c ? a : c;
+        y = a < c ? c : a;
     };
+    // cos and sin from h = (a_yy - a_xx) / 2 and g = a_xy: with 1/r =
+    // (h^2 + g^2)^(-1/2), cos^2 = (1 + |h|/r) / 2 and sin = sign(h) g / (2 r
+    // cos): two reciprocal square roots in a row instead of two square roots
+    // and three divisions
     auto rotation = [&](int x, int y, T& c, T& sn, T& tn) {
-        const T g = A[x][y];
+        const T g = A[x][y], h = T(0.5) * (A[y][y] - A[x][x]), r2 = h * h + g * g;
         c = T(1);
         sn = tn = T(0);
-        if (g != T(0)) {
-            const T th = (A[y][y] - A[x][x]) / (g + g);
-            tn = copysign(T(1) / (fabs(th) + sqrt(T(1) + th * th)), th);
-            c = T(1) / sqrt(T(1) + tn * tn);
-            sn = tn * c;
+        if (g != T(0) && r2 > T(0)) {
+            const T ir = rsqrt(r2), c2 = T(0.5) + T(0.5) * fabs(h) * ir, ic = rsqrt(c2);
+            c = c2 * ic;
+            sn = copysign(T(0.5) * ir * ic, h) * g;
+            tn = sn * ic;
         }
     };
     const int i = lane >> 3, k = lane & 7;
@@ -1046,7 +1061,7 @@ __global__ __launch_bounds__(64) void dc_leaf_kernel(const T* d, const T* e, con
             __syncthreads();
         }
         // a sweep that met only entries at rounding level has annihilated them
-        if (!(wave_max(off) > Eps<T>::v * scale)) break;
+        if (!(wave_max(off) > Eps<T>::v)) break;
     }
     // ascending order (pads beyond m excluded)
     if (lane < m) {
@@ -1056,7 +1071,7 @@ __global__ __launch_bounds__(64) void dc_leaf_kernel(const T* d, const T* e, con
             const T v = A[u][u];
             rank += (v < w || (v == w && u < lane)) ? 1 : 0;
         }
-        lam[(size_t)p * n + s + rank] = w;
+        lam[(size_t)p * n + s + rank] = ldexp(w, ex);
         T* q = Q + (size_t)p * n * n + s + (size_t)(s + rank) * n;
         for (int r = 0; r < m; r++) q[r] = V[r][lane];
     }
