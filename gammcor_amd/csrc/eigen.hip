@@ -325,15 +325,203 @@ __device__ inline Vec16<T> bld16(__amdgpu_buffer_rsrc_t r, int voff, int soff)
     return __builtin_bit_cast(Vec16<T>, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
 
+// SYMV of one column step on the lower triangle of the trailing matrix, over
+// the workgroup's own columns r > j: dot part A(r:, r)^T v(r:) -> y, scatter
+// part A(c, r) v(r), c > r -> u (LDS atomics).
+// (16-byte path: n a multiple of the vector width, A and v 16-byte aligned;
+// KV columns per wave, UV row chunks of 64 vectors in flight per lane)
+template <class T, int KV, int UV, bool DET>
+__device__ __forceinline__ void sytrd_symv_vec(T* A, int n, int j, int gi, int G, int nslots, const T* v, T* u, T* y,
+                                               T dsc)
+{
+    constexpr int VN = 16 / sizeof(T);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // 16-byte path: a wave takes KV consecutive owned columns; lane l
+    // reads rows c..c+VN-1 (c = chunk + VN*l) of each, UV chunks in
+    // flight.  The first chunk (diagonal block) is masked, the rest
+    // are not: every row there lies below all KV columns.
+    static_assert(SY_OB % KV == 0, "a column group must lie inside one unit");
+    // groups in snake order over the waves: group work falls with the row
+    for (int t = 0;; t++) {
+        const int qg = t * SY_WAVES + ((t & 1) ? SY_WAVES - 1 - wave : wave);
+        if (KV * qg >= nslots) break;
+        const int r0 = owned_row(KV * qg, gi, G);
+        if (r0 + KV - 1 <= j || r0 >= n) continue;
+        T vk[KV], s[KV];
+        const T* col[KV];
+#pragma unroll
+        for (int kk = 0; kk < KV; kk++) {
+            const int r = r0 + kk;
+            const bool okk = r > j && r < n;
+            vk[kk] = okk ? v[r] : T(0);
+            col[kk] = A + (size_t)(okk ? r : r0) * n;
+            s[kk] = 0;
+        }
+        const int base = r0 & ~63;
+        {
+            const int c = base + VN * lane;
+            if (c < n) {
+                const Vec16<T> vv = ld16(v + c);
+                T w[VN];
+#pragma unroll
+                for (int e = 0; e < VN; e++) w[e] = 0;
+#pragma unroll
+                for (int kk = 0; kk < KV; kk++) {
+                    const int r = r0 + kk;
+                    if (r > j && r < n) {
+                        const Vec16<T> a = ld16(col[kk] + c);
+#pragma unroll
+                        for (int e = 0; e < VN; e++) {
+                            const int row = c + e;
+                            if (row >= r) s[kk] += a.x[e] * vv.x[e];
+                            if (row > r) w[e] += a.x[e] * vk[kk];
+                        }
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < VN; e++)
+                    if (c + e > j && c + e > r0) scat<DET>(&u[c + e], w[e], dsc);
+            }
+        }
+        // rows below the diagonal block through one buffer descriptor
+        // over the group's KV columns (KV n elements from column r0);
+        // a column past n reads column r0 instead, as above
+        const int r0s = __builtin_amdgcn_readfirstlane(r0);
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            A + (size_t)r0s * n, 0, KV * n * (int)sizeof(T), BUF_WORD3);
+        int soff[KV];
+#pragma unroll
+        for (int kk = 0; kk < KV; kk++) soff[kk] = (r0s + kk < n ? kk : 0) * n * (int)sizeof(T);
+        int c = base + 64 * VN + VN * lane;
+        for (; c + (UV - 1) * 64 * VN < n; c += UV * 64 * VN) {
+            Vec16<T> a[UV][KV], vv[UV];
+#pragma unroll
+            for (int uu = 0; uu < UV; uu++) {
+#pragma unroll
+                for (int kk = 0; kk < KV; kk++)
+                    a[uu][kk] = bld16<T>(rs, (c + uu * 64 * VN) * (int)sizeof(T), soff[kk]);
+                vv[uu] = ld16(v + c + uu * 64 * VN);
+            }
+#pragma unroll
+            for (int uu = 0; uu < UV; uu++) {
+                T w[VN];
+#pragma unroll
+                for (int e = 0; e < VN; e++) w[e] = 0;
+#pragma unroll
+                for (int kk = 0; kk < KV; kk++)
+#pragma unroll
+                    for (int e = 0; e < VN; e++) {
+                        s[kk] += a[uu][kk].x[e] * vv[uu].x[e];
+                        w[e] += a[uu][kk].x[e] * vk[kk];
+                    }
+#pragma unroll
+                for (int e = 0; e < VN; e++) scat<DET>(&u[c + uu * 64 * VN + e], w[e], dsc);
+            }
+        }
+        for (; c < n; c += 64 * VN) {
+            const Vec16<T> vv = ld16(v + c);
+            T w[VN];
+#pragma unroll
+            for (int e = 0; e < VN; e++) w[e] = 0;
+#pragma unroll
+            for (int kk = 0; kk < KV; kk++) {
+                const Vec16<T> a = bld16<T>(rs, c * (int)sizeof(T), soff[kk]);
+#pragma unroll
+                for (int e = 0; e < VN; e++) {
+                    s[kk] += a.x[e] * vv.x[e];
+                    w[e] += a.x[e] * vk[kk];
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < VN; e++) scat<DET>(&u[c + e], w[e], dsc);
+        }
+        {
+            const T t = wave_sum_cols<KV>(s, lane);
+            const int kk = lane >> (6 - ilog2<KV>());
+            const int r = r0 + kk;
+            if ((lane & (64 / KV - 1)) == 0 && r > j && r < n) y[KV * qg + kk] = t;
+        }
+    }
+}
+// (any order and alignment)
+template <class T, bool DET>
+__device__ __forceinline__ void sytrd_symv_scalar(T* A, int n, int j, int gi, int G, int nslots, const T* v, T* u,
+                                                  T* y, T dsc)
+{
+    // columns per wave: FP32 halves the HBM time per element, so it groups
+    // columns to keep the LDS atomic unit off the critical path
+    constexpr int KC = sizeof(T) == 8 ? 1 : 4;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // each wave takes KC consecutive owned columns r0..r0+KC-1 (a unit
+    // holds SY_OB/KC such groups): one LDS atomic per row for their scatters
+    for (int t = 0;; t++) {
+        static_assert(SY_OB % KC == 0, "a column group must lie inside one unit");
+        const int qg = t * SY_WAVES + ((t & 1) ? SY_WAVES - 1 - wave : wave);
+        if (KC * qg >= nslots) break;
+        const int r0 = owned_row(KC * qg, gi, G);
+        if (r0 + KC - 1 <= j || r0 >= n) continue;
+        bool ok[KC];
+        T vk[KC], s[KC];
+        const T* col[KC];
+#pragma unroll
+        for (int kk = 0; kk < KC; kk++) {
+            const int r = r0 + kk;
+            ok[kk] = r > j && r < n;
+            vk[kk] = ok[kk] ? v[r] : T(0);
+            col[kk] = A + (size_t)(ok[kk] ? r : r0) * n;
+            s[kk] = 0;
+        }
+        if (KC == 1) {
+            // single column: four row chunks in flight per lane
+            T s1 = 0, s2 = 0, s3 = 0;
+            const T* c0p = col[0];
+            const T vr = vk[0];
+            int c = r0 + lane;
+            for (; c + 192 < n; c += 256) {
+                const T x0 = c0p[c], x1 = c0p[c + 64], x2 = c0p[c + 128], x3 = c0p[c + 192];
+                s[0] += x0 * v[c];
+                s1 += x1 * v[c + 64];
+                s2 += x2 * v[c + 128];
+                s3 += x3 * v[c + 192];
+                if (c > r0) scat<DET>(&u[c], x0 * vr, dsc);
+                scat<DET>(&u[c + 64], x1 * vr, dsc);
+                scat<DET>(&u[c + 128], x2 * vr, dsc);
+                scat<DET>(&u[c + 192], x3 * vr, dsc);
+            }
+            for (; c < n; c += 64) {
+                const T x0 = c0p[c];
+                s[0] += x0 * v[c];
+                if (c > r0) scat<DET>(&u[c], x0 * vr, dsc);
+            }
+            s[0] += (s1 + s2) + s3;
+        } else {
+            for (int c = r0 + lane; c < n; c += 64) {
+                // v[c] is only defined for c > j: touch it only under a valid column
+                T w = 0;
+#pragma unroll
+                for (int kk = 0; kk < KC; kk++) {
+                    if (ok[kk] && c >= r0 + kk) {
+                        const T a = col[kk][c];
+                        s[kk] += a * v[c];
+                        if (c > r0 + kk) w += a * vk[kk];
+                    }
+                }
+                if (c > j && c > r0) scat<DET>(&u[c], w, dsc);
+            }
+        }
+        {
+            const T t = wave_sum_cols<KC>(s, lane);
+            const int kk = lane >> (6 - ilog2<KC>());
+#pragma unroll
+            for (int k2 = 0; k2 < KC; k2++)
+                if (k2 == kk && (lane & (64 / KC - 1)) == 0 && ok[k2]) y[KC * qg + k2] = t;
+        }
+    }
+}
+
 template <class T, bool VLDS, bool PLDS, int KV, int UV, bool DET>
 __global__ __launch_bounds__(SY_THREADS) void sytrd_panel_kernel(PanelArgs<T> g)
 {
-    // columns per wave in the SYMV: FP32 halves the HBM time per element, so
-    // it groups columns to keep the LDS atomic unit off the critical path
-    constexpr int KC = sizeof(T) == 8 ? 1 : 4;
-    // 16-byte path (n a multiple of the vector width): KV columns per wave,
-    // UV row chunks of 64 vectors in flight per lane
-    constexpr int VN = 16 / sizeof(T);
     extern __shared__ char smem[];
     const int n = g.n, k = g.k, kb = g.kb, nb = g.nb, G = g.G;
     // Workgroups are dispatched round-robin over the 8 XCDs.  When G divides
@@ -466,180 +654,8 @@ __global__ __launch_bounds__(SY_THREADS) void sytrd_panel_kernel(PanelArgs<T> g)
         for (int c = tid; c < 2 * i; c += SY_THREADS) t12[c] = T(0);
         __syncthreads();
 
-        // SYMV on the lower triangle: dot part -> y, scatter part -> u (LDS atomics)
-        if (g.vec) {
-            // 16-byte path: a wave takes KV consecutive owned columns; lane l
-            // reads rows c..c+VN-1 (c = chunk + VN*l) of each, UV chunks in
-            // flight.  The first chunk (diagonal block) is masked, the rest
-            // are not: every row there lies below all KV columns.
-            static_assert(SY_OB % KV == 0, "a column group must lie inside one unit");
-            // groups in snake order over the waves: group work falls with the row
-            for (int t = 0;; t++) {
-                const int qg = t * SY_WAVES + ((t & 1) ? SY_WAVES - 1 - wave : wave);
-                if (KV * qg >= nslots) break;
-                const int r0 = owned_row(KV * qg, gi, G);
-                if (r0 + KV - 1 <= j || r0 >= n) continue;
-                T vk[KV], s[KV];
-                const T* col[KV];
-#pragma unroll
-                for (int kk = 0; kk < KV; kk++) {
-                    const int r = r0 + kk;
-                    const bool okk = r > j && r < n;
-                    vk[kk] = okk ? v[r] : T(0);
-                    col[kk] = A + (size_t)(okk ? r : r0) * n;
-                    s[kk] = 0;
-                }
-                const int base = r0 & ~63;
-                {
-                    const int c = base + VN * lane;
-                    if (c < n) {
-                        const Vec16<T> vv = ld16(v + c);
-                        T w[VN];
-#pragma unroll
-                        for (int e = 0; e < VN; e++) w[e] = 0;
-#pragma unroll
-                        for (int kk = 0; kk < KV; kk++) {
-                            const int r = r0 + kk;
-                            if (r > j && r < n) {
-                                const Vec16<T> a = ld16(col[kk] + c);
-#pragma unroll
-                                for (int e = 0; e < VN; e++) {
-                                    const int row = c + e;
-                                    if (row >= r) s[kk] += a.x[e] * vv.x[e];
-                                    if (row > r) w[e] += a.x[e] * vk[kk];
-                                }
-                            }
-                        }
-#pragma unroll
-                        for (int e = 0; e < VN; e++)
-                            if (c + e > j && c + e > r0) scat<DET>(&u[c + e], w[e], dsc);
-                    }
-                }
-                // rows below the diagonal block through one buffer descriptor
-                // over the group's KV columns (KV n elements from column r0);
-                // a column past n reads column r0 instead, as above
-                const int r0s = __builtin_amdgcn_readfirstlane(r0);
-                const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-                    A + (size_t)r0s * n, 0, KV * n * (int)sizeof(T), BUF_WORD3);
-                int soff[KV];
-#pragma unroll
-                for (int kk = 0; kk < KV; kk++) soff[kk] = (r0s + kk < n ? kk : 0) * n * (int)sizeof(T);
-                int c = base + 64 * VN + VN * lane;
-                for (; c + (UV - 1) * 64 * VN < n; c += UV * 64 * VN) {
-                    Vec16<T> a[UV][KV], vv[UV];
-#pragma unroll
-                    for (int uu = 0; uu < UV; uu++) {
-#pragma unroll
-                        for (int kk = 0; kk < KV; kk++)
-                            a[uu][kk] = bld16<T>(rs, (c + uu * 64 * VN) * (int)sizeof(T), soff[kk]);
-                        vv[uu] = ld16(v + c + uu * 64 * VN);
-                    }
-#pragma unroll
-                    for (int uu = 0; uu < UV; uu++) {
-                        T w[VN];
-#pragma unroll
-                        for (int e = 0; e < VN; e++) w[e] = 0;
-#pragma unroll
-                        for (int kk = 0; kk < KV; kk++)
-#pragma unroll
-                            for (int e = 0; e < VN; e++) {
-                                s[kk] += a[uu][kk].x[e] * vv[uu].x[e];
-                                w[e] += a[uu][kk].x[e] * vk[kk];
-                            }
-#pragma unroll
-                        for (int e = 0; e < VN; e++) scat<DET>(&u[c + uu * 64 * VN + e], w[e], dsc);
-                    }
-                }
-                for (; c < n; c += 64 * VN) {
-                    const Vec16<T> vv = ld16(v + c);
-                    T w[VN];
-#pragma unroll
-                    for (int e = 0; e < VN; e++) w[e] = 0;
-#pragma unroll
-                    for (int kk = 0; kk < KV; kk++) {
-                        const Vec16<T> a = bld16<T>(rs, c * (int)sizeof(T), soff[kk]);
-#pragma unroll
-                        for (int e = 0; e < VN; e++) {
-                            s[kk] += a.x[e] * vv.x[e];
-                            w[e] += a.x[e] * vk[kk];
-                        }
-                    }
-#pragma unroll
-                    for (int e = 0; e < VN; e++) scat<DET>(&u[c + e], w[e], dsc);
-                }
-                {
-                    const T t = wave_sum_cols<KV>(s, lane);
-                    const int kk = lane >> (6 - ilog2<KV>());
-                    const int r = r0 + kk;
-                    if ((lane & (64 / KV - 1)) == 0 && r > j && r < n) y[KV * qg + kk] = t;
-                }
-            }
-        } else
-        // each wave takes KC consecutive owned columns r0..r0+KC-1 (a unit
-        // holds SY_OB/KC such groups): one LDS atomic per row for their scatters
-        for (int t = 0;; t++) {
-            static_assert(SY_OB % KC == 0, "a column group must lie inside one unit");
-            const int qg = t * SY_WAVES + ((t & 1) ? SY_WAVES - 1 - wave : wave);
-            if (KC * qg >= nslots) break;
-            const int r0 = owned_row(KC * qg, gi, G);
-            if (r0 + KC - 1 <= j || r0 >= n) continue;
-            bool ok[KC];
-            T vk[KC], s[KC];
-            const T* col[KC];
-#pragma unroll
-            for (int kk = 0; kk < KC; kk++) {
-                const int r = r0 + kk;
-                ok[kk] = r > j && r < n;
-                vk[kk] = ok[kk] ? v[r] : T(0);
-                col[kk] = A + (size_t)(ok[kk] ? r : r0) * n;
-                s[kk] = 0;
-            }
-            if (KC == 1) {
-                // single column: four row chunks in flight per lane
-                T s1 = 0, s2 = 0, s3 = 0;
-                const T* c0p = col[0];
-                const T vr = vk[0];
-                int c = r0 + lane;
-                for (; c + 192 < n; c += 256) {
-                    const T x0 = c0p[c], x1 = c0p[c + 64], x2 = c0p[c + 128], x3 = c0p[c + 192];
-                    s[0] += x0 * v[c];
-                    s1 += x1 * v[c + 64];
-                    s2 += x2 * v[c + 128];
-                    s3 += x3 * v[c + 192];
-                    if (c > r0) scat<DET>(&u[c], x0 * vr, dsc);
-                    scat<DET>(&u[c + 64], x1 * vr, dsc);
-                    scat<DET>(&u[c + 128], x2 * vr, dsc);
-                    scat<DET>(&u[c + 192], x3 * vr, dsc);
-                }
-                for (; c < n; c += 64) {
-                    const T x0 = c0p[c];
-                    s[0] += x0 * v[c];
-                    if (c > r0) scat<DET>(&u[c], x0 * vr, dsc);
-                }
-                s[0] += (s1 + s2) + s3;
-            } else {
-                for (int c = r0 + lane; c < n; c += 64) {
-                    // v[c] is only defined for c > j: touch it only under a valid column
-                    T w = 0;
-#pragma unroll
-                    for (int kk = 0; kk < KC; kk++) {
-                        if (ok[kk] && c >= r0 + kk) {
-                            const T a = col[kk][c];
-                            s[kk] += a * v[c];
-                            if (c > r0 + kk) w += a * vk[kk];
-                        }
-                    }
-                    if (c > j && c > r0) scat<DET>(&u[c], w, dsc);
-                }
-            }
-            {
-                const T t = wave_sum_cols<KC>(s, lane);
-                const int kk = lane >> (6 - ilog2<KC>());
-#pragma unroll
-                for (int k2 = 0; k2 < KC; k2++)
-                    if (k2 == kk && (lane & (64 / KC - 1)) == 0 && ok[k2]) y[KC * qg + k2] = t;
-            }
-        }
+        if (g.vec) sytrd_symv_vec<T, KV, UV, DET>(A, n, j, gi, G, nslots, v, u, y, dsc);
+        else sytrd_symv_scalar<T, DET>(A, n, j, gi, G, nslots, v, u, y, dsc);
         __syncthreads();
         if constexpr (DET) {
             // the fixed-point scatter sums back to T
@@ -807,6 +823,7 @@ __global__ __launch_bounds__(SY_THREADS) void sytrd_panel_kernel(PanelArgs<T> g)
 }
 
 #include "sytrd_resident.hpp"
+#include "sytrd_xpanel.hpp"
 
 // After the last panel: d[n-1], and clear everything on/above the diagonal so
 // the strictly lower triangle holds the unit-lower reflectors.
@@ -1750,8 +1767,12 @@ static int eig_layout(EigPlan<T>* p, char* base)
     take(p->e, B * n * sizeof(T));
     take(p->tau, B * n * sizeof(T));
     take(p->part, B * (2 + G * (2 + 2 * nb)) * sizeof(T));
-    take(p->Pu, B * G * n * sizeof(T));
-    take(p->vg, B * G * n * sizeof(T));
+    // (the exchange words of sytrd_xpanel_kernel's scatter sums, or the scatter
+    // sums and the copies of v of sytrd_panel_kernel)
+    take(p->Pu, 2 * B * G * n * sizeof(T));
+    p->vg = base ? p->Pu + B * G * n : nullptr;
+    take(p->xa, B * n * 2 * sizeof(T) * 2);
+    take(p->xd, B * G * 2 * nb * sizeof(T) * 2);
     take(p->Q, B * nn * sizeof(T));
     take(p->QK, B * nn * sizeof(T));
     take(p->QN, B * nn * sizeof(T));
@@ -2024,7 +2045,36 @@ int syevd_batched(hipStream_t s, EigPlan<T>& p, T* A, T* w)
         }
         // (set by an eager call before a capture; not repeated inside one)
         if (!capturing(s)) GMC_HIP(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        unsigned epoch = 0;
+        // panels with their exchanges in words: the 16-byte SYMV, v in LDS, rows
+        // of exchange A in registers, and rows of the trailing matrix for every
+        // workgroup to the panel's end (16 G of them: two full rounds of units).
+        // In FP64 every workgroup's reading of exchange A, 32 bytes a row, ends
+        // the gain at about 19 MB per column over all workgroups (panels,
+        // barriers -> words: 2144 x 32 112 -> 103 ms, 2664 x 8 69.7 -> 70.1,
+        // 4524 x 16 445 -> 449; FP32 79 -> 63, 61 -> 45, 299 -> 254)
+        const int vec = (n % (16 / (int)sizeof(T)) == 0) && (reinterpret_cast<uintptr_t>(A) % 16 == 0) &&
+                        (reinterpret_cast<uintptr_t>(p.vg) % 16 == 0);
+        const bool xpl = xp_lds<T>(n, nslots_max, nb, true) <= LDS_MAX;
+        const size_t xlds = xp_lds<T>(n, nslots_max, nb, xpl);
+        auto xpanel = [&](int k, int kb) {
+            return vec && n <= XP_C * SY_THREADS && xlds <= LDS_MAX && n - k - kb >= 2 * SY_OB * G &&
+                   (sizeof(T) == 4 || (int64_t)B * G * n <= 600000);
+        };
+        const void* xfn = det ? (xpl ? (const void*)sytrd_xpanel_kernel<T, true, KV, UV, true>
+                                     : (const void*)sytrd_xpanel_kernel<T, false, KV, UV, true>)
+                              : (xpl ? (const void*)sytrd_xpanel_kernel<T, true, KV, UV, false>
+                                     : (const void*)sytrd_xpanel_kernel<T, false, KV, UV, false>);
+        if (n > p.mres && xpanel(0, std::min(nb, n - 1))) {
+            if (!capturing(s))
+                GMC_HIP(hipFuncSetAttribute(xfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)xlds));
+            const int64_t wb = (int64_t)B * G * n * sizeof(T) / 2, wa = (int64_t)B * n * sizeof(T),
+                          wd = (int64_t)B * G * 2 * nb * sizeof(T) / 2;
+            hipLaunchKernelGGL(zero_u32, dim3((unsigned)((wb + 255) / 256)), dim3(256), 0, s, (unsigned*)p.Pu, (int)wb);
+            hipLaunchKernelGGL(zero_u32, dim3((unsigned)((wa + 255) / 256)), dim3(256), 0, s, (unsigned*)p.xa, (int)wa);
+            hipLaunchKernelGGL(zero_u32, dim3((unsigned)((wd + 255) / 256)), dim3(256), 0, s, (unsigned*)p.xd, (int)wd);
+            GMC_HIP(hipGetLastError());
+        }
+        unsigned epoch = 0, xepoch = 0;
         for (int k = 0; k < n - 1; k += nb) {
             if (n - k <= p.mres) {
                 // the rest fits in the register files: one resident launch,
@@ -2046,18 +2096,21 @@ int syevd_batched(hipStream_t s, EigPlan<T>& p, T* A, T* w)
                 break;
             }
             const int kb = std::min(nb, n - 1 - k);
-            const int vec = (n % (16 / (int)sizeof(T)) == 0) && (reinterpret_cast<uintptr_t>(A) % 16 == 0) &&
-                            (reinterpret_cast<uintptr_t>(p.vg) % 16 == 0);
             PanelArgs<T> a{A, p.W, p.X, p.d, p.e, p.tau, p.part, p.Pu, p.vg, p.bar, p.err, p.fro, n, k, kb, nb, G,
                            epoch, vec};
-            void* args[] = {&a};
+            XPanelArgs<T> xargs{A, p.W, p.X, p.d, p.e, p.tau, reinterpret_cast<unsigned long long*>(p.xa),
+                                reinterpret_cast<unsigned long long*>(p.Pu), reinterpret_cast<unsigned long long*>(p.xd),
+                                p.err, p.fro, n, k, kb, nb, G, xepoch};
+            const bool xp = xpanel(k, kb);
+            void* args[] = {xp ? (void*)&xargs : (void*)&a};
             double bytes = 0.0;   // lower triangle of the trailing matrix, once per column
             for (int jj = k; jj < k + kb; jj++) bytes += 0.5 * (double)(n - jj - 1) * (double)(n - jj) * sizeof(T);
             {
                 ProfScope ps(s, sizeof(T) == 8 ? "sytrd_panel_f64" : "sytrd_panel_f32", bytes * B);
-                GMC_TRY(launch_persistent(kfn, dim3(B * G), dim3(SY_THREADS), args, lds, s));
+                GMC_TRY(launch_persistent(xp ? xfn : kfn, dim3(B * G), dim3(SY_THREADS), args, xp ? xlds : lds, s));
             }
-            epoch += 2 * kb;   // two group barriers per column
+            if (xp) xepoch += kb;      // one epoch per column
+            else epoch += 2 * kb;      // two group barriers per column
             const int k1 = k + kb;
             if (k1 < n) {
                 const int mt = n - k1;

@@ -164,7 +164,7 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
             }
             s1 = wave_total(s1);
             if (lane == 0) redA[wave] = s1;
-            __syncthreads();
+            lds_barrier();
             s1 = T(0);
             for (int i = 0; i < nwave; i++) s1 += redA[i];
             // a2 = -tau/2 w^T v, w' = w + a2 v, column j less v w'(j) + w' v(j), v(j) = 1
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
         }
         nrm = wave_total(nrm);
         if (lane == 0) redB[wave] = nrm;
-        __syncthreads();
+        lds_barrier();
         // the reflector
         T xn2 = 0;
         for (int i = 0; i < nwave; i++) xn2 += redB[i];

@@ -7,6 +7,16 @@
 
 namespace gmc {
 
+// Workgroup barrier for data in LDS only.  __syncthreads also waits for the
+// waves' outstanding global accesses, stores included: after a store that has
+// to travel to memory (an exchange between workgroups) that is 2-4 us.
+__device__ inline void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // v of lane l (uniform), as a scalar.
 __device__ inline float read_lane(float v, int l)
 {
