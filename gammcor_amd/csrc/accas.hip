@@ -18,6 +18,7 @@
 #include "chol.hpp"
 #include "oa_policy.hpp"
 #include "gemm.hpp"
+#include "negeig.hpp"
 #include "prof.hpp"
 #include "wave_ops.hpp"
 
@@ -822,6 +823,47 @@ __global__ __launch_bounds__(64) void sum_partials_kernel(const double* partial,
     if (threadIdx.x == 0) W[b] = s + *wdiag;
 }
 
+// Products with a Cholesky factor L (lower triangular) over TRI_SLICES
+// slices that skip its zero triangle: A- L by column slices (columns [c0, c1)
+// need rows c0.. of L), L^T T by row slices of the lower triangle (rows [r0,
+// r1) need rows r0.. of T and columns up to r1), L Z by row slices (rows [r0,
+// r1) need columns up to r1 of L): 9/16, 15/64 and 9/16 of the full products.
+constexpr int TRI_SLICES = 8;
+static int tri_cut(int n, int p) { return (int)((int64_t)n * p / TRI_SLICES); }
+// M = L^T Am L, its lower triangle (and what lies in the slices above it),
+// through T = Am L; M may take Am's place.
+static int factor_m(hipStream_t st, int n, int B, const double* L, const double* Am, double* T, double* M)
+{
+    const int64_t snn = (int64_t)n * n;
+    for (int p = 0; p < TRI_SLICES; p++) {
+        const int c0 = tri_cut(n, p), c1 = tri_cut(n, p + 1);
+        if (c1 <= c0) continue;
+        GemmShape g{n, c1 - c0, n - c0, false, false, n, n, n, snn, snn, snn, B, 0};
+        GMC_TRY(gemm_big<double>(st, g, 1.0, Am + (size_t)c0 * n, L + c0 + (size_t)c0 * n, 0.0, T + (size_t)c0 * n));
+    }
+    for (int p = 0; p < TRI_SLICES; p++) {
+        const int r0 = tri_cut(n, p), r1 = tri_cut(n, p + 1);
+        if (r1 <= r0) continue;
+        GemmShape g{r1 - r0, r1, n - r0, true, false, n, n, n, snn, snn, snn, B, 0};
+        GMC_TRY(gemm_big<double>(st, g, 1.0, L + r0 + (size_t)r0 * n, T + r0, 0.0, M + r0));
+    }
+    return 0;
+}
+// Y = L Z.
+static int factor_y(hipStream_t st, int n, int B, const double* L, const double* Z, double* Y)
+{
+    const int64_t snn = (int64_t)n * n;
+    for (int p = 0; p < TRI_SLICES; p++) {
+        const int r0 = tri_cut(n, p), r1 = tri_cut(n, p + 1);
+        if (r1 <= r0) continue;
+        GemmShape g{r1 - r0, n, r1, false, false, n, n, n, snn, snn, snn, B, 0};
+        GMC_TRY(gemm_big<double>(st, g, 1.0, L + r0, Z, 0.0, Y + r0));
+    }
+    return 0;
+}
+
+__global__ void pad_diag_set_kernel(const BatchSys* sys, int nalpha, double* A, int npad, double sign);
+
 template <class T>
 int erpa_plan(int n, int batch, ErpaPlan<T>* p)
 {
@@ -829,15 +871,16 @@ int erpa_plan(int n, int batch, ErpaPlan<T>* p)
     p->batch = batch;
     const size_t nn = (size_t)n * n;
     const size_t mat = batch * nn * sizeof(T), vec = batch * n * sizeof(T);
+    const size_t fac = sizeof(T) == 8 && n >= NEGEIG_MIN ? negeig_bytes(n, batch) : 0;
     p->ws_bytes = carve_bytes({mat, mat, mat, mat, vec, vec, batch * sizeof(double),
-                               (size_t)batch * 1024 * sizeof(double)});
+                               (size_t)batch * 1024 * sizeof(double), fac});
     return 0;
 }
 
 template <class T>
 int erpa_batched(hipStream_t st, ErpaPlan<T>& p, const AbPair& ab, const double* alphas, int nalpha,
                  const double* Gw, const double* wdiag, void* scratch, ErpaOut& out, double* Y_out, double* S_out,
-                 double* Am_out, const ErpaBatchTables* bt)
+                 double* Am_out, const ErpaBatchTables* bt, const EigSolveAt* factor_eig, void* ws, size_t ws_bytes)
 {
     GMC_CHECK(nalpha >= 1 && nalpha <= p.batch, "ERPA: %d alpha points for a plan of %d", nalpha, p.batch);
     GMC_CHECK(p.eig && p.eig->bound && p.eig->batch == p.batch && p.eig->n == p.n, "ERPA: eigensolver plan unbound");
@@ -853,24 +896,30 @@ int erpa_batched(hipStream_t st, ErpaPlan<T>& p, const AbPair& ab, const double*
     double* d_al = ar.take<double>(p.batch);
     const int npart = 1024;
     double* partial = ar.take<double>((size_t)p.batch * npart);
+    const size_t fac_bytes = sizeof(T) == 8 && n >= NEGEIG_MIN ? negeig_bytes(n, p.batch) : 0;
+    char* fac = ar.take<char>(fac_bytes);
     GMC_CHECK(ar.fits(), "ERPA: scratch layout overflow");
     const int nprob = bt ? bt->nsys * nalpha : nalpha;   // problems of this call
     GMC_CHECK(nprob <= p.batch, "ERPA: %d problems for a plan of %d", nprob, p.batch);
-    hipLaunchKernelGGL(zero_int_kernel, dim3((nprob + 255) / 256), dim3(256), 0, st, out.nneg, nprob);
 
     const dim3 blk(256);
-    // A+(alpha) -> E, A-(alpha) -> Tb
     const int nt64f = (n + 63) / 64;
-    if (bt) {
-        // the batching form: alphas are already on the device
-        hipLaunchKernelGGL(form_pad_kernel<T>, form_grid(nt64f * (nt64f + 1) / 2, bt->nsys, nalpha), blk, 0, st, bt->sys,
-                           bt->nsys, alphas, nalpha, E, Tb, n);
-    } else {
-        GMC_HIP(hipMemcpyAsync(d_al, alphas, nalpha * sizeof(double), hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(form_kernel<T>, form_grid(nt64f * (nt64f + 1) / 2, 1, B), blk, 0, st, ab.p0, ab.p1, ab.m0, ab.m1,
-                           d_al, B, E, Tb, n);
-    }
-    GMC_HIP(hipGetLastError());
+    if (!bt) GMC_HIP(hipMemcpyAsync(d_al, alphas, nalpha * sizeof(double), hipMemcpyHostToDevice, st));
+    // A+(alpha) -> E, A-(alpha) -> Tb
+    auto form = [&]() -> int {
+        hipLaunchKernelGGL(zero_int_kernel, dim3((nprob + 255) / 256), dim3(256), 0, st, out.nneg, nprob);
+        if (bt) {
+            // the batching form: alphas are already on the device
+            hipLaunchKernelGGL(form_pad_kernel<T>, form_grid(nt64f * (nt64f + 1) / 2, bt->nsys, nalpha), blk, 0, st,
+                               bt->sys, bt->nsys, alphas, nalpha, E, Tb, n);
+        } else {
+            hipLaunchKernelGGL(form_kernel<T>, form_grid(nt64f * (nt64f + 1) / 2, 1, B), blk, 0, st, ab.p0, ab.p1,
+                               ab.m0, ab.m1, d_al, B, E, Tb, n);
+        }
+        GMC_HIP(hipGetLastError());
+        return 0;
+    };
+    GMC_TRY(form());
     const int Bp = nprob;   // the solve below runs over every problem
     const dim3 gsq((n + 255) / 256, n, Bp);
     if (Am_out) {
@@ -879,30 +928,56 @@ int erpa_batched(hipStream_t st, ErpaPlan<T>& p, const AbPair& ab, const double*
     }
     EigPlan<T>& ep = *p.eig;
     GMC_CHECK(ep.batch == Bp, "ERPA: plan batch %d != %d problems", ep.batch, Bp);
-    GMC_TRY(syevd_batched<T>(st, ep, E, lam));
-    hipLaunchKernelGGL(sqrt_scale_kernel<T>, gsq, blk, 0, st, E, lam, n, out.nneg);
-    GMC_HIP(hipGetLastError());
-    // S = V|L|^(1/2)V^T
-    // S is symmetric: its lower triangle, mirrored
-    GemmShape gS{n, n, n, false, true, n, n, n, (int64_t)nn, (int64_t)nn, (int64_t)nn, Bp, 1};
-    GMC_TRY(gemm_big<T>(st, gS, T(1), E, E, T(0), Sb));
     const int nt64 = (n + 63) / 64;
-    hipLaunchKernelGGL(mirror_lower_kernel<T>, dim3(nt64, nt64, Bp), blk, 0, st, Sb, n);
-    if (S_out) {
-        GMC_CHECK(sizeof(T) == 8, "ERPA: A+^(1/2) output is available from the FP64 solve");
-        GMC_HIP(hipMemcpyAsync(S_out, Sb, Bp * nn * sizeof(T), hipMemcpyDeviceToDevice, st));
-    }
-    // M = S A- S
     GemmShape gN{n, n, n, false, false, n, n, n, (int64_t)nn, (int64_t)nn, (int64_t)nn, Bp, 0};
-    GMC_TRY(gemm_big<T>(st, gN, T(1), Tb, Sb, T(0), Mb));
-    GemmShape gNl = gN;
-    gNl.uplo = 1;   // M is symmetric: its lower triangle, mirrored
-    GMC_TRY(gemm_big<T>(st, gNl, T(1), Sb, Mb, T(0), Tb));
+    // a factor F of |A+| = F F^T: its Cholesky factor L, or S = |A+|^(1/2)
+    // (the reference's; M = F^T A- F and Y = F Z are the same but for a
+    // rotation that Z carries, see the Cholesky route below)
+    bool chol = false;
+    if constexpr (sizeof(T) == 8) {
+        hipStreamCaptureStatus cst = hipStreamCaptureStatusNone;
+        GMC_HIP(hipStreamIsCapturing(st, &cst));
+        if (factor_eig && !S_out && n >= NEGEIG_MIN && cst == hipStreamCaptureStatusNone) {
+            // (padded modes of the batching form: A+ needs them above zero; L's
+            // are sqrt of that, M's are zero as below)
+            if (bt) hipLaunchKernelGGL(pad_diag_set_kernel, dim3(Bp), blk, 0, st, bt->sys, nalpha, E, n, 1.0);
+            GMC_TRY(abs_factor(st, n, Bp, E, Mb, Sb, fac, fac_bytes, out.nneg, *factor_eig, ws, ws_bytes,
+                               getenv("GMC_OA_STATS") != nullptr, &chol));
+            if (!chol) GMC_TRY(form());
+        }
+        if (chol) {
+            // M (-> Tb, lower triangle) through Sb; the mirror below
+            GMC_TRY(factor_m(st, n, Bp, E, Tb, Sb, Tb));
+        }
+    }
+    if (!chol) {
+        GMC_TRY(syevd_batched<T>(st, ep, E, lam));
+        hipLaunchKernelGGL(sqrt_scale_kernel<T>, gsq, blk, 0, st, E, lam, n, out.nneg);
+        GMC_HIP(hipGetLastError());
+        // S = V|L|^(1/2)V^T
+        // S is symmetric: its lower triangle, mirrored
+        GemmShape gS{n, n, n, false, true, n, n, n, (int64_t)nn, (int64_t)nn, (int64_t)nn, Bp, 1};
+        GMC_TRY(gemm_big<T>(st, gS, T(1), E, E, T(0), Sb));
+        hipLaunchKernelGGL(mirror_lower_kernel<T>, dim3(nt64, nt64, Bp), blk, 0, st, Sb, n);
+        if (S_out) {
+            GMC_CHECK(sizeof(T) == 8, "ERPA: A+^(1/2) output is available from the FP64 solve");
+            GMC_HIP(hipMemcpyAsync(S_out, Sb, Bp * nn * sizeof(T), hipMemcpyDeviceToDevice, st));
+        }
+        // M = S A- S
+        GMC_TRY(gemm_big<T>(st, gN, T(1), Tb, Sb, T(0), Mb));
+        GemmShape gNl = gN;
+        gNl.uplo = 1;   // M is symmetric: its lower triangle, mirrored
+        GMC_TRY(gemm_big<T>(st, gNl, T(1), Sb, Mb, T(0), Tb));
+    }
     hipLaunchKernelGGL(mirror_lower_kernel<T>, dim3(nt64, nt64, Bp), blk, 0, st, Tb, n);
     GMC_HIP(hipGetLastError());
     GMC_TRY(syevd_batched<T>(st, ep, Tb, om2));
-    // Y = S Z
-    GMC_TRY(gemm_big<T>(st, gN, T(1), Sb, Tb, T(0), Mb));
+    // Y = F Z
+    if (chol) {
+        if constexpr (sizeof(T) == 8) GMC_TRY(factor_y(st, n, Bp, E, Tb, Mb));
+    } else {
+        GMC_TRY(gemm_big<T>(st, gN, T(1), Sb, Tb, T(0), Mb));
+    }
     hipLaunchKernelGGL(ycols_kernel<T>, gsq, blk, 0, st, Mb, E, om2, out.eig, n);
     GMC_HIP(hipGetLastError());
     // P = Yf Yf^T (lower) and W (skipped without integrand weights)
@@ -2112,12 +2187,27 @@ int erpa_batched_mixed(hipStream_t st, EigPlan<float>& ep, int n, const AbPair& 
         hipLaunchKernelGGL(form_kernel<double>, form_grid(nt64f * (nt64f + 1) / 2, 1, B), blk, 0, st, ab.p0, ab.p1, ab.m0,
                            ab.m1, d_al, B, Ap, Am, n);
     }
-    // eig(A+) in FP32, refined in FP64
-    hipLaunchKernelGGL(f64_to_f32_kernel, dim3(gcopy), blk, 0, st, Ap, E32, (int64_t)B * nn);
-    GMC_HIP(hipGetLastError());
-    GMC_TRY(syevd_batched<float>(st, ep, E32, w32));
-    hipLaunchKernelGGL(f32_to_f64_kernel, dim3(gcopy), blk, 0, st, E32, X, (int64_t)B * nn);
-    GMC_HIP(hipGetLastError());
+    const char* route = getenv("GMC_MIXED_ROUTE");
+    const bool want_chol = !(route && strcmp(route, "eigen") == 0);
+    // Large orders: |A+|'s factor from the pairs below zero alone, which a
+    // Krylov basis gives in a fraction of A+'s eigensolve (negeig.hpp)
+    bool chol_ok = false;
+    if (want_chol && cluster_eig && n >= NEGEIG_MIN && negeig_bytes(n, B) <= B * nn * sizeof(float)) {
+        ProfScope ps(st, "mixed_chol_route", 0.0);
+        GMC_HIP(hipMemcpyAsync(AX, Ap, (size_t)B * nn * sizeof(double), hipMemcpyDeviceToDevice, st));
+        GMC_TRY(abs_factor(st, n, B, AX, X, Xn, E32, B * nn * sizeof(float), out.nneg, *cluster_eig, Sb,
+                           reinterpret_cast<char*>(Gb + B * nn) - reinterpret_cast<char*>(Sb), stats, &chol_ok));
+        if (!chol_ok)
+            hipLaunchKernelGGL(zero_int_kernel, dim3((B + 255) / 256), dim3(256), 0, st, out.nneg, B);
+    }
+    if (!chol_ok) {
+        // eig(A+) in FP32, refined in FP64
+        hipLaunchKernelGGL(f64_to_f32_kernel, dim3(gcopy), blk, 0, st, Ap, E32, (int64_t)B * nn);
+        GMC_HIP(hipGetLastError());
+        GMC_TRY(syevd_batched<float>(st, ep, E32, w32));
+        hipLaunchKernelGGL(f32_to_f64_kernel, dim3(gcopy), blk, 0, st, E32, X, (int64_t)B * nn);
+        GMC_HIP(hipGetLastError());
+    }
     const int nt64 = (n + 63) / 64;
     // The Cholesky route: L L^T = |A+| into AX.  ok stays false when the
     // restricted refinement does not reach OAC_TOL in OAC_MAX_STEPS steps or a
@@ -2181,9 +2271,7 @@ int erpa_batched_mixed(hipStream_t st, EigPlan<float>& ep, int n, const AbPair& 
         ok = true;
         return 0;
     };
-    bool chol_ok = false;
-    const char* route = getenv("GMC_MIXED_ROUTE");
-    if (!(route && strcmp(route, "eigen") == 0)) GMC_TRY(chol_route(chol_ok));
+    if (want_chol && !chol_ok) GMC_TRY(chol_route(chol_ok));
     if (!chol_ok) {
         // the eigen route of the reference: A+ refined in full, S = V|L|^(1/2)V^T (into AX)
         ProfScope ps(st, "mixed_eigen_route", 0.0);
@@ -2196,30 +2284,11 @@ int erpa_batched_mixed(hipStream_t st, EigPlan<float>& ep, int n, const AbPair& 
         GMC_TRY(gemm_big<double>(st, gS, 1.0, X, X, 0.0, AX));
         hipLaunchKernelGGL(mirror_lower_kernel<double>, dim3(nt64, nt64, B), blk, 0, st, AX, n);
     }
-    // M = F^T A- F (into Ap) for the factor F in AX (L, or S = S^T).  With L
-    // the products run over TRI_SLICES slices that skip its zero triangle:
-    // A- L by column slices (columns [c0, c1) need rows c0.. of L), L^T Sb
-    // by row slices of the lower triangle (rows [r0, r1) need rows r0.. of
-    // Sb and columns up to r1), L Z by row slices (rows [r0, r1) need
-    // columns up to r1 of L): 9/16, 15/64 and 9/16 of the full products.
+    // M = F^T A- F (into Ap) for the factor F in AX (L, or S = S^T)
     const int64_t snn = (int64_t)nn;
-    constexpr int TRI_SLICES = 8;
-    auto cut = [&](int p) { return (int)((int64_t)n * p / TRI_SLICES); };
     GemmShape gN{n, n, n, false, false, n, n, n, snn, snn, snn, B, 0};
     if (chol_ok) {
-        for (int p = 0; p < TRI_SLICES; p++) {
-            const int c0 = cut(p), c1 = cut(p + 1);
-            if (c1 <= c0) continue;
-            GemmShape g{n, c1 - c0, n - c0, false, false, n, n, n, snn, snn, snn, B, 0};
-            GMC_TRY(gemm_big<double>(st, g, 1.0, Am + (size_t)c0 * n, AX + c0 + (size_t)c0 * n, 0.0,
-                                     Sb + (size_t)c0 * n));
-        }
-        for (int p = 0; p < TRI_SLICES; p++) {
-            const int r0 = cut(p), r1 = cut(p + 1);
-            if (r1 <= r0) continue;
-            GemmShape g{r1 - r0, r1, n - r0, true, false, n, n, n, snn, snn, snn, B, 0};
-            GMC_TRY(gemm_big<double>(st, g, 1.0, AX + r0 + (size_t)r0 * n, Sb + r0, 0.0, Ap + r0));
-        }
+        GMC_TRY(factor_m(st, n, B, AX, Am, Sb, Ap));
     } else {
         GMC_TRY(gemm_big<double>(st, gN, 1.0, Am, AX, 0.0, Sb));
         GemmShape gTl{n, n, n, true, false, n, n, n, snn, snn, snn, B, 1};
@@ -2253,12 +2322,7 @@ int erpa_batched_mixed(hipStream_t st, EigPlan<float>& ep, int n, const AbPair& 
     }
     // Y = F Z (Sb), filtered copy (Gb), P = Yf Yf^T (Am), integrand
     if (chol_ok) {
-        for (int p = 0; p < TRI_SLICES; p++) {
-            const int r0 = cut(p), r1 = cut(p + 1);
-            if (r1 <= r0) continue;
-            GemmShape g{r1 - r0, n, r1, false, false, n, n, n, snn, snn, snn, B, 0};
-            GMC_TRY(gemm_big<double>(st, g, 1.0, AX + r0, X, 0.0, Sb + r0));
-        }
+        GMC_TRY(factor_y(st, n, B, AX, X, Sb));
     } else {
         GMC_TRY(gemm_big<double>(st, gN, 1.0, AX, X, 0.0, Sb));
     }
@@ -2280,9 +2344,11 @@ int erpa_batched_mixed(hipStream_t st, EigPlan<float>& ep, int n, const AbPair& 
 template int erpa_plan<double>(int, int, ErpaPlan<double>*);
 template int erpa_plan<float>(int, int, ErpaPlan<float>*);
 template int erpa_batched<double>(hipStream_t, ErpaPlan<double>&, const AbPair&, const double*, int, const double*,
-                                  const double*, void*, ErpaOut&, double*, double*, double*, const ErpaBatchTables*);
+                                  const double*, void*, ErpaOut&, double*, double*, double*, const ErpaBatchTables*, const EigSolveAt*,
+                                  void*, size_t);
 template int erpa_batched<float>(hipStream_t, ErpaPlan<float>&, const AbPair&, const double*, int, const double*,
-                                 const double*, void*, ErpaOut&, double*, double*, double*, const ErpaBatchTables*);
+                                 const double*, void*, ErpaOut&, double*, double*, double*, const ErpaBatchTables*, const EigSolveAt*,
+                                  void*, size_t);
 
 // ------------------------------------------------------------ integrand from given Y
 // Columns of Y whose Eig lies in (1e-3, 1e8) (acfd.f:4976, 5013), others zero.

@@ -48,6 +48,11 @@ struct ErpaOut {
     int* nneg = nullptr;      // device, nalpha: negative eigenvalues of A+
 };
 
+// FP64 eigensolve of nb problems of order m side by side (stride m*m,
+// overwritten by their eigenvectors; w gets the eigenvalues, ascending) in
+// the caller's workspace ws of ws_bytes bytes (eig_workspace_bytes).
+using EigSolveAt = std::function<int(double* A, double* w, int m, int nb, void* ws, size_t ws_bytes)>;
+
 template <class T>
 struct ErpaPlan {
     int n = 0, batch = 0;
@@ -80,10 +85,15 @@ int erpa_plan(int n, int batch, ErpaPlan<T>* p);
 // alpha points, each system's matrices padded to the plan's order (ab, Gw and
 // wdiag unused; alphas then on the device); the padded modes are decoupled
 // and carry no integrand weight.
+// With factor_eig (FP64, an eigensolver that runs in the plan's own
+// workspace ws) orders from NEGEIG_MIN up take a Cholesky factor of |A+| in
+// place of S (abs_factor, negeig.hpp) unless S_out asks for S itself; it
+// decides on the host, so not while a graph is captured.
 template <class T>
 int erpa_batched(hipStream_t st, ErpaPlan<T>& p, const AbPair& ab, const double* alphas, int nalpha,
                  const double* Gw, const double* wdiag, void* scratch, ErpaOut& out, double* Y_out = nullptr,
-                 double* S_out = nullptr, double* Am_out = nullptr, const ErpaBatchTables* bt = nullptr);
+                 double* S_out = nullptr, double* Am_out = nullptr, const ErpaBatchTables* bt = nullptr,
+                 const EigSolveAt* factor_eig = nullptr, void* ws = nullptr, size_t ws_bytes = 0);
 
 // W = sum Gw o (Yf Yf^T) + wdiag for a given normalised Y and Eig (ACEneERPA,
 // acfd.f:4968-5043), Yf the columns with 1e-3 < Eig < 1e8.
@@ -126,10 +136,6 @@ constexpr float OAC_TOL = 1e-11f;
 // FP64 eigensolve of nb problems side by side (stride n*n, overwritten by
 // their eigenvectors; w gets the eigenvalues, ascending).
 using EigSolve64 = std::function<int(double* A, double* w, int nb)>;
-// FP64 eigensolve of nb problems of order m side by side (stride m*m,
-// overwritten by their eigenvectors; w gets the eigenvalues, ascending) in
-// the caller's workspace ws of ws_bytes bytes (eig_workspace_bytes).
-using EigSolveAt = std::function<int(double* A, double* w, int m, int nb, void* ws, size_t ws_bytes)>;
 
 // Mixed path: FP32 eigen solves refined by n_min to n_max Ogita-Aishima
 // steps in FP64 (more than n_min while the corrections stay at or above

@@ -211,8 +211,10 @@ int gmc_acecorr_batch_dev(int prec, int nsys, const int* nbasis, const int* nina
             GMC_TRY(erpa_plan<double>(npad, B, &pl));
             pl.eig = ep;
             GMC_TRY(st.erpaws.reserve(align_up(pl.ws_bytes)));
+            const EigSolveAt factor_eig = st.eig_at(s);
             GMC_TRY(erpa_batched<double>(s, pl, none, d_al, nalpha, nullptr, nullptr, st.erpaws.ptr, outs[g], nullptr,
-                                         nullptr, nullptr, &bt));
+                                         nullptr, nullptr, &bt, graph ? nullptr : &factor_eig, st.scratch.ptr,
+                                         ep->ws_bytes));
             if (check) {
                 GMC_TRY(eig_check_error<double>(s, *ep));
             } else {

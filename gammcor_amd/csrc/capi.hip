@@ -245,7 +245,10 @@ int ac_alpha_batches(hipStream_t s, AcRun& r, int prec, int cap, int nalpha, con
                 pl.eig = ep;
                 GMC_TRY(st.erpaws.reserve(align_up(pl.ws_bytes) + outb));
                 bind_out(align_up(pl.ws_bytes));
-                GMC_TRY(erpa_batched<T>(s, pl, r.ab, alphas + a0, B, r.Gw, r.wdiag, st.erpaws.ptr, out, nullptr));
+                const EigSolveAt factor_eig = st.eig_at(s);
+                GMC_TRY(erpa_batched<T>(s, pl, r.ab, alphas + a0, B, r.Gw, r.wdiag, st.erpaws.ptr, out, nullptr, nullptr,
+                                        nullptr, nullptr, prec == GMC_FP64 ? &factor_eig : nullptr, st.scratch.ptr,
+                                        ep->ws_bytes));
                 GMC_TRY(eig_check_error<T>(s, *ep));
                 return 0;
             };

@@ -252,7 +252,9 @@ static int erpa_one_fp64(hipStream_t s, int n, const AbPair& ab, double alpha, c
     out.W = reinterpret_cast<double*>(base);
     out.eig = reinterpret_cast<double*>(base + align_up(8));
     out.nneg = reinterpret_cast<int*>(base + align_up(8) + align_up((size_t)n * 8));
-    GMC_TRY(erpa_batched<double>(s, pl, ab, &alpha, 1, Gw, wdiag, st.erpaws.ptr, out, d_Y, d_S, d_Am));
+    const EigSolveAt factor_eig = st.eig_at(s);
+    GMC_TRY(erpa_batched<double>(s, pl, ab, &alpha, 1, Gw, wdiag, st.erpaws.ptr, out, d_Y, d_S, d_Am, nullptr,
+                                 d_Y ? nullptr : &factor_eig, st.scratch.ptr, ep->ws_bytes));
     GMC_TRY(eig_check_error<double>(s, *ep));
     if (eig_host) GMC_HIP(hipMemcpyAsync(eig_host, out.eig, (size_t)n * 8, hipMemcpyDeviceToHost, s));
     if (W_host && Gw) GMC_HIP(hipMemcpyAsync(W_host, out.W, 8, hipMemcpyDeviceToHost, s));

@@ -6,6 +6,7 @@
 #include <tuple>
 #include <vector>
 
+#include "accas.hpp"
 #include "chol.hpp"
 #include "common.hpp"
 #include "eigen.hpp"
@@ -47,6 +48,12 @@ struct State {
     // (eig_workspace_bytes<double>(n, nb) bytes): the mixed path's large
     // refinement clusters
     int solve64_at(hipStream_t s, int n, double* A, double* w, int nb, void* ws, size_t ws_bytes);
+    EigSolveAt eig_at(hipStream_t s)
+    {
+        return [this, s](double* A, double* w, int m, int nb, void* ws, size_t wsb) {
+            return solve64_at(s, m, A, w, nb, ws, wsb);
+        };
+    }
     // The batching form's last captured FP64 group sequence: replayed while
     // its key (sizes, alphas, groups, workspace address) and the workspace
     // generation are unchanged.
