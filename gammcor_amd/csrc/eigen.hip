@@ -2082,12 +2082,12 @@ int syevd_batched(hipStream_t s, EigPlan<T>& p, T* A, T* w)
                 // (its two group barriers) at every order that fits
                 const int m = n - k;
                 const ResShape rs = res_shape(m, B, p.ncu);
-                const size_t words = (size_t)B * 2 * m * res_words<T>() * 2;   // of 32 bits
-                GMC_CHECK(rs.R > 0 && words * 4 <= (size_t)B * n * 3 * nb * sizeof(T), "syevd: resident shape");
-                ResArgs<T> ra{A, p.d, p.e, p.tau, reinterpret_cast<unsigned long long*>(p.X), p.err, n, k, rs.G};
+                const void* rk = res_kernel<T>(rs);
+                const size_t words = (size_t)B * RES_RING * res_buf(rs.G, rs.R) * (sizeof(T) / 4);   // of 32 bits
+                GMC_CHECK(rk && words * 4 <= (size_t)B * n * 3 * nb * sizeof(T), "syevd: resident shape");
+                ResArgs<T> ra{A, p.d, p.e, p.tau, p.X, p.err, n, k, rs.G};
                 void* rargs[] = {&ra};
-                const void* rk = res_kernel<T>(rs.R, rs.C);
-                const size_t rl = res_lds<T>(m, rs.R);
+                const size_t rl = res_lds<T>(m, rs);
                 if (!capturing(s)) GMC_HIP(hipFuncSetAttribute(rk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)rl));
                 hipLaunchKernelGGL(zero_u32, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s,
                                    reinterpret_cast<unsigned*>(p.X), (int)words);

@@ -1,83 +1,188 @@
 // Tridiagonalisation of trailing problems that fit in the register files of
-// the GPU: one persistent launch holds the whole matrix in registers and
-// applies every rank-2 update at once (no panels, no trailing products).
-// Workgroup gi of a problem keeps the rows gi, gi + G, ... (at most R of
-// them), thread t their columns t, t + blockDim, ... (at most C), both
-// triangles.
+// the GPU: one persistent launch holds the whole matrix in registers, both
+// triangles, and applies every rank-2 update at once (no panels, no trailing
+// products).  Workgroup gi of a problem keeps the rows gi, gi + G, ...
 //
-// What bounds it is the latency of one exchange per column, so there is only
-// one: each workgroup publishes, for its own rows r, w_r = tau (A v)_r and
-// a_r = A(r, j+1), and every workgroup forms a2, w' = w + a2 v, column j+1 of
-// the updated matrix and its reflector redundantly from them, then updates
-// and multiplies its own rows.  (The panel kernel's lower-triangle SYMV
-// needs two exchanges: its scatter sums must be collected before w exists.)
-// A value travels in 8-byte words of 32 data bits and the column's epoch,
-// stored and polled as relaxed agent-scope atomics: no flag, no fence and no
-// cache-wide write-back, the words themselves say when they are there.  Two
-// buffers suffice: a workgroup publishes epoch e + 2 only after it has read
-// every row's e + 1, which each owner publishes after it has read e; a
-// workgroup whose rows are all done has nothing left to read and leaves.
+// What bounds it is the latency of a column's chain (publish, read, reductions,
+// update and product), so there is one exchange and one barrier per column,
+// made of what the owners have before the reflector is known: for its own rows
+// r a workgroup publishes S_r = (A xt)_r (xt: the column's tail) and a_r = A(r,
+// j+1).  While these travel everyone forms the reflector v = scal xt + e(j+1)
+// from its own copy of the column; then, from the words, w = tau A v = tau (scal
+// S + a), w^T v, w' = w - tau/2 (w^T v) v and column j+1 of the updated matrix,
+// and updates and multiplies its own rows.
+//
+// A word that is not there yet is zero, and a zero is published as -0: the
+// words are stored and polled at agent scope and need no flag and no fence (a
+// flag per column and the data behind it are two trips; words with an epoch
+// beside 32 data bits are twice the traffic).  Four buffers: publishing epoch e,
+// a wave also clears its words of epoch e - 2, which everyone had read before
+// publishing e - 1, whose words this workgroup has read; the clearing store is
+// complete (vmcnt) before the same wave publishes e + 1, and nobody polls for e
+// + 2 in that buffer before it has read e + 1.  A workgroup whose rows are all
+// done has nothing left to read and leaves.
+//
+// Two layouts of a workgroup's rows over its threads: up to order 512 each
+// wave has whole rows (sytrd_resident_rows_kernel: a row's product is one wave's
+// sum, reduced columns and rows are skipped, but every wave forms the whole
+// column, which costs more than it saves from there on), above each thread has
+// some columns of every row (sytrd_resident_kernel).
 //
 // Every sum is formed in a fixed order, so the result does not depend on
 // timing (it serves the deterministic mode as it is).
 //
-// Measured, tridiagonalisation alone, panels and trailing updates -> here:
-//   order x problems    410 x 8        1281 x 1        2048 x 1        1024 x 8
-//   FP64             6.7 -> 1.4 ms  23.5 -> 5.3 ms  39.3 -> 9.2 ms  20.7 -> 4.8 ms
-//   FP32             7.0 -> 1.1 ms  25.7 -> 4.4 ms  45.9 -> 7.2 ms  22.2 -> 3.5 ms
-// 3.3 us per column at order 410, about half of it the exchange; the FP64
-// update and product of R C elements per thread are most of the rest at 2048.
+// Measured, tridiagonalisation alone in FP64: panels and trailing updates -> one
+// exchange per column with two barriers, reflector before publication -> here
+//   order x problems   256 x 64     410 x 8       1024 x 8      1281 x 1      2048 x 1
+//   ms                3.4 1.2 0.78  6.7 1.4 0.97  20.7 4.8 4.04 23.5 5.3 3.75 39.3 9.2 6.79
+// 1.8 us per column at order 85, 2.4 at 410, 2.9 at 1281 (a word's way from one
+// compute unit to another: 0.3 to 0.4 us).
 //
 // Included by eigen.hip only, inside its namespace.
 #pragma once
 
 constexpr int RES_THREADS = 512, RES_WAVES = RES_THREADS / 64;
-constexpr int RES_CH = 16;   // own rows whose products are reduced together
-constexpr int RES_WAIT = 14;   // pause before a column's first poll, in units of 64 clocks
+constexpr int RES_CH = 16;    // own rows whose products are reduced together
+constexpr int RES_WAIT = 2;   // pause before a column's first poll, in units of 64 clocks
+constexpr int RES_RING = 4;   // buffers of the exchange
+constexpr int RES_PG = 4;     // workgroups per problem / 64, at most
+constexpr int RES_ROWS_MAX = 512;   // order up to which a wave has whole rows
 
 template <class T>
 struct ResArgs {
     T *A, *d, *e, *tau;
-    unsigned long long* ring;   // per problem 2 buffers x m rows x res_words, zero on entry
+    T* ring;                  // per problem RES_RING x res_buf elements, zero on entry
     int* err;
-    int n, j0, G;               // order (ld and stride of A, d, e, tau), first column, workgroups per problem
+    int n, j0, G;             // order (ld and stride of A, d, e, tau), first column, workgroups per problem
 };
 
-// Words of one row's (w, a).
-template <class T>
-constexpr int res_words() { return 2 * (int)(sizeof(T) / 4); }
+// Elements of one exchange buffer: (S, a) of every position (gi R + q for row q
+// of workgroup gi), then every workgroup's share of xt^T A xt (to 16 bytes).
+constexpr int res_buf(int G, int R) { return 2 * G * R + (G + 3) / 4 * 4; }
 
-// Half h of a row's packet (0: w, 1: a).
-__device__ inline void res_put(unsigned long long* q, int h, float x, unsigned ep)
-{
-    const unsigned long long t = (unsigned long long)ep << 32;
-    __hip_atomic_store(q + h, t | __float_as_uint(x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline void res_put(unsigned long long* q, int h, double x, unsigned ep)
-{
-    const unsigned long long t = (unsigned long long)ep << 32, b = (unsigned long long)__double_as_longlong(x);
-    __hip_atomic_store(q + 2 * h, t | (b & 0xffffffffull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(q + 2 * h + 1, t | (b >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline void res_unpack(const unsigned long long (&x)[2], float& w, float& a)
-{
-    w = __uint_as_float((unsigned)x[0]);
-    a = __uint_as_float((unsigned)x[1]);
-}
-__device__ inline void res_unpack(const unsigned long long (&x)[4], double& w, double& a)
-{
-    w = __longlong_as_double((long long)((x[1] << 32) | (x[0] & 0xffffffffull)));
-    a = __longlong_as_double((long long)((x[3] << 32) | (x[2] & 0xffffffffull)));
-}
-// Dynamic LDS of the kernel for a trailing order m.
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// Agent-scope words of a buffer (byte offsets): a pair (S, a) and one value.
+// A value's word or half of a pair is never +0 once published.
 template <class T>
-constexpr size_t res_lds(int m, int R) { return ((size_t)m + 2 * RES_WAVES + 4 + 2 * R + (size_t)RES_WAVES * R) * sizeof(T); }
+struct ResRing;
+template <>
+struct ResRing<double> {
+    static constexpr int SC1 = 16;   // cache policy: agent scope
+    typedef u32x4 pair;
+    typedef u32x2 word;
+    static __device__ inline pair get2(__amdgpu_buffer_rsrc_t r, int o) { return __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, SC1); }
+    static __device__ inline word get1(__amdgpu_buffer_rsrc_t r, int o) { return __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, SC1); }
+    static __device__ inline void put2(__amdgpu_buffer_rsrc_t r, int o, pair p) { __builtin_amdgcn_raw_buffer_store_b128(p, r, o, 0, SC1); }
+    static __device__ inline void put1(__amdgpu_buffer_rsrc_t r, int o, word p) { __builtin_amdgcn_raw_buffer_store_b64(p, r, o, 0, SC1); }
+    static __device__ inline bool there(pair p) { return (p.x | p.y) != 0 && (p.z | p.w) != 0; }
+    static __device__ inline bool there(word p) { return (p.x | p.y) != 0; }
+    static __device__ inline double val(word p)
+    {
+        return __longlong_as_double((long long)(((unsigned long long)p.y << 32) | p.x));
+    }
+    static __device__ inline double first(pair p) { return val(word{p.x, p.y}); }
+    static __device__ inline double second(pair p) { return val(word{p.z, p.w}); }
+    static __device__ inline word bits(double x)
+    {
+        const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+        const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+        return word{lo, (lo | hi) == 0 ? 0x80000000u : hi};
+    }
+    static __device__ inline pair bits(double x, double y)
+    {
+        const word a = bits(x), b = bits(y);
+        return pair{a.x, a.y, b.x, b.y};
+    }
+};
+template <>
+struct ResRing<float> {
+    static constexpr int SC1 = 16;
+    typedef u32x2 pair;
+    typedef unsigned word;
+    static __device__ inline pair get2(__amdgpu_buffer_rsrc_t r, int o) { return __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, SC1); }
+    static __device__ inline word get1(__amdgpu_buffer_rsrc_t r, int o) { return __builtin_amdgcn_raw_buffer_load_b32(r, o, 0, SC1); }
+    static __device__ inline void put2(__amdgpu_buffer_rsrc_t r, int o, pair p) { __builtin_amdgcn_raw_buffer_store_b64(p, r, o, 0, SC1); }
+    static __device__ inline void put1(__amdgpu_buffer_rsrc_t r, int o, word p) { __builtin_amdgcn_raw_buffer_store_b32(p, r, o, 0, SC1); }
+    static __device__ inline bool there(pair p) { return p.x != 0 && p.y != 0; }
+    static __device__ inline bool there(word p) { return p != 0; }
+    static __device__ inline float val(word p) { return __uint_as_float(p); }
+    static __device__ inline float first(pair p) { return __uint_as_float(p.x); }
+    static __device__ inline float second(pair p) { return __uint_as_float(p.y); }
+    static __device__ inline word bits(float x)
+    {
+        const unsigned b = __float_as_uint(x);
+        return b == 0 ? 0x80000000u : b;
+    }
+    static __device__ inline pair bits(float x, float y) { return pair{bits(x), bits(y)}; }
+};
+
+// 1 / x to rounding level: the hardware's estimate and two Newton steps (the
+// IEEE division's scaling and fix-up are as long again, on the critical path).
+__device__ inline double res_rcp(double x)
+{
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+__device__ inline float res_rcp(float x) { return 1.0f / x; }
+
+// The sum of the waves' values x[0], x[stride], ...: all loads at once, as a
+// tree (a loop over the waves there are waits for each load: 700 cycles of 8).
+template <class T>
+__device__ inline T res_wave_sum(const T* x, int stride)
+{
+    T s[RES_WAVES];
+#pragma unroll
+    for (int w = 0; w < RES_WAVES; w++) s[w] = x[w * stride];
+#pragma unroll
+    for (int h = RES_WAVES / 2; h >= 1; h /= 2)
+#pragma unroll
+        for (int w = 0; w < h; w++) s[w] += s[w + h];
+    return s[0];
+}
+// The sum over each group of R neighbouring lanes.
+template <int R, class T>
+__device__ inline T res_group_total(T v)
+{
+    v += dpp_mov<DPP_XOR1>(v);
+    v += dpp_mov<DPP_XOR2>(v);
+    v += dpp_mov<DPP_HALF_MIRROR>(v);
+    if constexpr (R >= 16) v += dpp_mov<DPP_MIRROR>(v);
+    if constexpr (R >= 32) v = swap_add<16>(v, v);
+    if constexpr (R >= 64) v = swap_add<32>(v, v);
+    return v;
+}
+
+// A bounded poll's end: every 64th pass, whether some workgroup has given up,
+// and after 2^21 passes (seconds: a lost workgroup) giving up.
+__device__ inline bool res_give_up(long spins, int* err, int lane)
+{
+    if ((spins & 63) != 63) return false;
+    if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return true;
+    if (spins <= (1L << 21)) return false;
+    if (lane == 0) atomicExch(err, 1);
+    return true;
+}
+
+// Thread t keeps the columns at the positions t, t + blockDim, ... (at most C)
+// of R rows: what a wave reads of the exchange is contiguous.  The sum of xt^T A
+// xt travels as a share per workgroup: a sum over the column's waves would be a
+// second barrier.
+// Dynamic LDS for a trailing order m (everything twice: a
+// column's writes need no barrier behind the last column's reads).
+template <class T>
+constexpr size_t res_lds(int m, int R)
+{
+    return 2 * ((size_t)m + RES_WAVES + 4 + R + (size_t)RES_WAVES * R) * sizeof(T);
+}
 
 template <class T, int R, int C>
 __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> g)
 {
-    constexpr int NW = res_words<T>();
-    constexpr int CH = R < RES_CH ? R : RES_CH, NCH = R / CH;
+    typedef ResRing<T> Ring;
+    constexpr int CH = R < RES_CH ? R : RES_CH, NCH = R / CH, ES = (int)sizeof(T);
     extern __shared__ char smem[];
     const int n = g.n, m = g.n - g.j0, G = g.G;
     // (a problem's workgroups on one XCD where G allows it, as in the panel kernel)
@@ -85,116 +190,160 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
     const int lin = (nwg % 8 == 0 && (nwg / 8) % G == 0) ? (int)(blockIdx.x & 7) * (nwg / 8) + (int)(blockIdx.x >> 3)
                                                       : (int)blockIdx.x;
     const int p = lin / G, gi = lin % G;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, NT = blockDim.x, nwave = NT >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, NT = blockDim.x;
     T* A = g.A + (size_t)p * n * n + g.j0 + (size_t)g.j0 * n;   // the trailing matrix, ld n
-    unsigned long long* ring = g.ring + (size_t)p * 2 * m * NW;
+    const int bufb = res_buf(G, R) * ES, share = 2 * G * R * ES;
+    const __amdgpu_buffer_rsrc_t ring = __builtin_amdgcn_make_buffer_rsrc(
+        g.ring + (size_t)p * RES_RING * res_buf(G, R), 0, RES_RING * bufb, 0x20000);   // (32-bit elements, no stride)
     T* dd = g.d + (size_t)p * n + g.j0;
     T* ee = g.e + (size_t)p * n + g.j0;
     T* tt = g.tau + (size_t)p * n + g.j0;
-    T* lx = reinterpret_cast<T*>(smem);   // m: column j
-    T* redA = lx + m;                     // RES_WAVES
-    T* redB = redA + RES_WAVES;           // RES_WAVES
-    T* sc = redB + RES_WAVES;             // [0] w(j) [1] x(j) [2] x(j+1)
-    T* acol = sc + 4;                     // R: own rows' entries of column j+1
-    T* wown = acol + R;                   // R: own rows' w
-    T* part = wown + R;                   // RES_WAVES x R: the waves' parts of own rows' products
+    T* lx0 = reinterpret_cast<T*>(smem);        // 2 x m: column j
+    T* redB0 = lx0 + 2 * m;                     // 2 x RES_WAVES
+    T* sc0 = redB0 + 2 * RES_WAVES;             // 2 x 4: [0] x(j) [1] x(j+1)
+    T* acol0 = sc0 + 8;                         // 2 x R: own rows' entries of column j+1
+    T* part0 = acol0 + 2 * R;                   // 2 x RES_WAVES x R: the waves' parts of own rows' products
 
-    T a[R][C], v[C], x[C], vown[NCH];
+    // (the sums over waves run over RES_WAVES of them)
+    for (int i = tid; i < 2 * RES_WAVES; i += NT) redB0[i] = T(0);
+    for (int i = tid; i < 2 * RES_WAVES * R; i += NT) part0[i] = T(0);
+    lds_barrier();
+
+    T a[R][C], v[C], x[C], vown[NCH], wown[NCH];
+    int col[C];   // (m: none)
+#pragma unroll
+    for (int k = 0; k < C; k++) {
+        const int pos = tid + k * NT, c = (pos % R) * G + pos / R;
+        col[k] = pos < G * R && c < m ? c : m;
+    }
 #pragma unroll
     for (int q = 0; q < R; q++) {
         const int r = q * G + gi;
 #pragma unroll
         for (int k = 0; k < C; k++) {
-            const int c = tid + k * NT;
+            const int c = col[k];
             a[q][k] = r < m && c < m ? (c >= r ? A[c + (size_t)r * n] : A[r + (size_t)c * n]) : T(0);
         }
     }
     // column 0 arrives final
 #pragma unroll
     for (int k = 0; k < C; k++) {
-        const int c = tid + k * NT;
         v[k] = T(0);
-        x[k] = c < m ? A[c] : T(0);
+        x[k] = col[k] < m ? A[col[k]] : T(0);
     }
 #pragma unroll
-    for (int h = 0; h < NCH; h++) vown[h] = T(0);
+    for (int h = 0; h < NCH; h++) vown[h] = wown[h] = T(0);
     const int rlast = gi < m ? (m - 1 - gi) / G * G + gi : -1;   // last own row
-    T tau = 0;
-    for (int j = 0; j < m - 1 && rlast > j; j++) {
+    T tau = 0, scal = 0, beta = 0;
+    // column j's reflector into A, d, e and tau, by the owner of row j + 1, a
+    // step later: the stores' way to memory is then beside the arithmetic, and
+    // column 0 is overwritten only when every workgroup has loaded its rows
+    auto store_reflector = [&](int j) {
+        if ((j + 1) % G != gi) return;
+        const T* lx = lx0 + (j & 1) * m;
+        if (tid == 0) {
+            dd[j] = sc0[4 * (j & 1)];
+            ee[j] = beta;
+            tt[j] = tau;
+        }
+        for (int c = tid; c < m; c += NT)
+            if (c > j) A[c + (size_t)j * n] = c == j + 1 ? T(1) : scal * lx[c];
+    };
+    int j = 0, jg = 0, jq = 0;   // j = jq G + jg
+    for (; j < m - 1 && rlast > j; j++) {
+        T* lx = lx0 + (j & 1) * m;
+        T* redB = redB0 + (j & 1) * RES_WAVES;
+        T* sc = sc0 + 4 * (j & 1);
+        T* acol = acol0 + (j & 1) * R;
+        T* part = part0 + (j & 1) * RES_WAVES * R;
         T wp[C], a2 = 0;
 #pragma unroll
         for (int k = 0; k < C; k++) wp[k] = T(0);
         if (j > 0) {
-            // w of column j - 1 and the entries of column j from their owners.
-            // The words take longer than RES_WAIT to arrive, and polls that
-            // fail delay them for everyone (8 problems of order 410: 2.9 ms
-            // polled at once, 1.36 ms with a pause of 12 to 16, 1.53 ms with 32)
+            // S and a of the rows from j on, row j's own, and the shares
             __builtin_amdgcn_s_sleep(RES_WAIT);
-            const unsigned long long* buf = ring + (size_t)(j & 1) * m * NW;
-            T wc[C], ac[C], s1 = 0;
+            const int base = (j & (RES_RING - 1)) * bufb;
+            // (each load under its own condition, so they go out one after the
+            // other; all at once is slower, 1281 x 1 3.8 -> 4.4 ms: at these
+            // orders everyone's reading is what the words wait for, and the
+            // pass then starts before they can have arrived)
+            typename Ring::pair pk[C], pj = Ring::bits(T(0), T(0));
+            typename Ring::word ps[RES_PG];
+            bool need[C], needj = true, needs[RES_PG];
+            const int oj = base + 2 * ES * (jg * R + jq);
 #pragma unroll
             for (int k = 0; k < C; k++) {
-                const int c = tid + k * NT;
-                wc[k] = ac[k] = T(0);
-                if (c >= j && c < m) {
-                    unsigned long long q[NW];
-                    const unsigned long long* src = buf + (size_t)c * NW;
-                    for (long spins = 0;; spins++) {
-                        bool ok = true;
-#pragma unroll
-                        for (int i = 0; i < NW; i++)
-                            q[i] = __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-                        for (int i = 0; i < NW; i++) ok = ok && (unsigned)(q[i] >> 32) == (unsigned)j;
-                        if (ok) break;
-                        if ((spins & 63) == 63) {
-                            if (__hip_atomic_load(g.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) break;
-                            if (spins > (1L << 21)) {   // seconds of polling: a lost workgroup
-                                atomicExch(g.err, 1);
-                                break;
-                            }
-                        }
-                    }
-                    res_unpack(q, wc[k], ac[k]);
-                    if (c == j) sc[0] = wc[k];
-                } else {
-                    v[k] = T(0);
-                }
-                s1 += wc[k] * v[k];
+                pk[k] = Ring::bits(T(0), T(0));
+                need[k] = col[k] >= j && col[k] < m;
             }
-            s1 = wave_total(s1);
-            if (lane == 0) redA[wave] = s1;
-            lds_barrier();
-            s1 = T(0);
-            for (int i = 0; i < nwave; i++) s1 += redA[i];
-            // a2 = -tau/2 w^T v, w' = w + a2 v, column j less v w'(j) + w' v(j), v(j) = 1
-            a2 = T(-0.5) * tau * s1;
-            const T wj = sc[0] + a2;
+#pragma unroll
+            for (int i = 0; i < RES_PG; i++) {
+                const int gq = lane + 64 * i;
+                ps[i] = Ring::bits(T(0));
+                needs[i] = gq < G && (m - 1 - gq) / G * G + gq >= j;
+            }
+            for (long spins = 0;; spins++) {
+                asm volatile("" ::: "memory");   // (every pass loads anew)
+#pragma unroll
+                for (int k = 0; k < C; k++)
+                    if (need[k]) pk[k] = Ring::get2(ring, base + 2 * ES * (tid + k * NT));
+                if (needj) pj = Ring::get2(ring, oj);
+#pragma unroll
+                for (int i = 0; i < RES_PG; i++)
+                    if (needs[i]) ps[i] = Ring::get1(ring, base + share + ES * (lane + 64 * i));
+                bool more = false;
+#pragma unroll
+                for (int k = 0; k < C; k++) {
+                    need[k] = need[k] && !Ring::there(pk[k]);
+                    more = more || need[k];
+                }
+                needj = needj && !Ring::there(pj);
+                more = more || needj;
+#pragma unroll
+                for (int i = 0; i < RES_PG; i++) {
+                    needs[i] = needs[i] && !Ring::there(ps[i]);
+                    more = more || needs[i];
+                }
+                if (__builtin_amdgcn_ballot_w64(more) == 0 || res_give_up(spins, g.err, lane)) break;
+            }
+            store_reflector(j - 1);
+            // xt^T A xt, then w^T v = tau (scal^2 xt^T A xt + 2 scal S(j) + a(j)):
+            // xt^T a = S(j) by symmetry
+            T q = Ring::val(ps[0]);
+#pragma unroll
+            for (int i = 1; i < RES_PG; i++) q += Ring::val(ps[i]);
+            q = wave_total(q);
+            const T Sj = Ring::first(pj), aj = Ring::second(pj);
+            a2 = T(-0.5) * tau * tau * (scal * (scal * q + T(2) * Sj) + aj);
+            // w' = w + a2 v, column j less v w'(j) + w' v(j), v(j) = 1
+            const T wj = tau * (scal * Sj + aj) + a2;
 #pragma unroll
             for (int k = 0; k < C; k++) {
-                wp[k] = wc[k] + a2 * v[k];
-                x[k] = ac[k] - v[k] * wj - wp[k];
+                const bool in = col[k] >= j && col[k] < m;
+                const T ak = in ? Ring::second(pk[k]) : T(0);
+                if (!in) v[k] = T(0);
+                wp[k] = in ? tau * (scal * Ring::first(pk[k]) + ak) + a2 * v[k] : T(0);
+                x[k] = ak - v[k] * wj - wp[k];
             }
         }
         // the column: its head, and the tail's entries xt with their norm
         T nrm = 0, xt[C];
 #pragma unroll
         for (int k = 0; k < C; k++) {
-            const int c = tid + k * NT;
+            const int c = col[k];
             xt[k] = c > j + 1 && c < m ? x[k] : T(0);
             nrm += xt[k] * xt[k];
-            if (c == j) sc[1] = x[k];
-            if (c == j + 1) sc[2] = x[k];
+            if (c == j) sc[0] = x[k];
+            if (c == j + 1 && c < m) sc[1] = x[k];
             if (c < m) lx[c] = x[k];
         }
         // own rows: the last column's rank-2 update and the product with the
-        // tail (v = scal xt + e_j+1 follows from it once the reflector is
-        // known), RES_CH rows at a time; finished rows are skipped by fours
+        // tail, RES_CH rows at a time; finished rows are skipped by fours
 #pragma unroll
         for (int h = 0; h < NCH; h++) {
             const int q0 = h * CH;
             // row q0 + l in lane l (< CH)
-            const T vr_l = vown[h], wr_l = j > 0 ? wown[q0 + (lane & (CH - 1))] + a2 * vr_l : T(0);
+            const T vr_l = vown[h], wr_l = wown[h] + a2 * vr_l;
             T acc[CH];
 #pragma unroll
             for (int q = 0; q < CH; q++) acc[q] = T(0);
@@ -213,7 +362,7 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
             }
 #pragma unroll
             for (int k = 0; k < C; k++)
-                if (tid + k * NT == j + 1) {
+                if (col[k] == j + 1) {
 #pragma unroll
                     for (int q = 0; q < CH; q++) acol[q0 + q] = a[q0 + q][k];
                 }
@@ -224,64 +373,324 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
         nrm = wave_total(nrm);
         if (lane == 0) redB[wave] = nrm;
         lds_barrier();
+        if (wave == 0 && j < m - 2) {
+            // publish; the words of two columns ago become free
+            const int base = ((j + 1) & (RES_RING - 1)) * bufb, old = ((j + 3) & (RES_RING - 1)) * bufb;
+            const int q = lane % R, r = q * G + gi, o = 2 * ES * (gi * R + q);
+            const T s = res_wave_sum(part + q, R);
+            const bool in = r > j && r < m, on = lane < R && in;
+            __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the last column's clearing stores are complete
+            if (on) Ring::put2(ring, base + o, Ring::bits(s, acol[q]));
+            const T t = res_group_total<R>(in && r > j + 1 ? s * lx[r] : T(0));
+            if (lane == 0) Ring::put1(ring, base + share + ES * gi, Ring::bits(t));
+            if (on) Ring::put2(ring, old + o, typename Ring::pair(0));
+            if (lane == 0) Ring::put1(ring, old + share + ES * gi, typename Ring::word(0));
+        }
         // the reflector
-        T xn2 = 0;
-        for (int i = 0; i < nwave; i++) xn2 += redB[i];
-        const T alpha = sc[2];
-        T beta = alpha, scal = 0;
-        tau = 0;
+        const T xn2 = res_wave_sum(redB, 1);
+        const T alpha = sc[1];
+        beta = alpha;
+        scal = tau = 0;
         if (xn2 != T(0)) {
-            beta = -copysign(sqrt(alpha * alpha + xn2), alpha);
-            tau = (beta - alpha) / beta;
-            scal = T(1) / (alpha - beta);
+            // |beta| = sqrt(s) = s rsqrt(s), tau = (beta - alpha) / beta, scal = 1 / (alpha - beta)
+            const T s = alpha * alpha + xn2, rs = rsqrt(s);
+            T b = s * rs;
+            b += T(0.5) * rs * fma(-b, b, s);
+            beta = -copysign(b, alpha);
+            tau = T(1) + fabs(alpha) * rs;
+            scal = res_rcp(alpha - beta);
         }
-        if (j < m - 2) {
-            unsigned long long* buf = ring + (size_t)((j + 1) & 1) * m * NW;
-            for (int i = tid; i < 2 * R; i += NT) {
-                const int q = i % R, h = i / R, r = q * G + gi;
-                T val = acol[q];
-                if (h == 0) {
-                    T s = 0;
-                    for (int w = 0; w < nwave; w++) s += part[w * R + q];
-                    val = tau * (scal * s + val);
-                    wown[q] = val;
-                }
-                if (r > j && r < m) res_put(buf + (size_t)r * NW, h, val, (unsigned)(j + 1));
-            }
-        }
-        // the owner of row j + 1 stores the reflector (column 0 waits for
-        // step 1: by then every workgroup has loaded its rows)
-        const bool writer = (j + 1) % G == gi;
-        if (writer && tid == 0) {
-            dd[j] = sc[1];
-            ee[j] = beta;
-            tt[j] = tau;
-            // the last diagonal element (sytrd_finish_kernel moves it to d)
-            if (j == m - 2) A[(size_t)(m - 1) * n + m - 1] = acol[(m - 1) / G];
-        }
+        if (j == m - 2 && tid == 0)   // the last diagonal element (sytrd_finish_kernel moves it to d)
+            A[(size_t)(m - 1) * n + m - 1] = acol[(m - 1) / G];
 #pragma unroll
-        for (int k = 0; k < C; k++) {
-            const int c = tid + k * NT;
-            if (writer && j == 1 && c >= 1 && c < m) A[c] = v[k];
-            v[k] = c == j + 1 ? T(1) : scal * xt[k];
-            if (writer && c > j && c < m && (j > 0 || m == 2)) A[c + (size_t)j * n] = v[k];
-        }
+        for (int k = 0; k < C; k++) v[k] = col[k] == j + 1 ? T(1) : scal * xt[k];
 #pragma unroll
         for (int h = 0; h < NCH; h++) {
-            const int r = (h * CH + (lane & (CH - 1))) * G + gi;
+            const int q = h * CH + (lane & (CH - 1)), r = q * G + gi;
+            const T s = res_wave_sum(part + q, R);
             vown[h] = r == j + 1 ? T(1) : (r > j + 1 && r < m ? scal * lx[r] : T(0));
+            wown[h] = tau * (scal * s + acol[q]);
         }
+        if (++jg == G) {
+            jg = 0;
+            jq++;
+        }
+    }
+    if (j > 0) store_reflector(j - 1);
+}
+
+// The sums over the wave of RW values per lane: the lane gets that of row lane
+// >> (6 - log2 RW).
+template <int RW, class T>
+__device__ inline T res_row_sums(T (&s)[RW], int lane)
+{
+    if constexpr (RW == 2) {
+        T t = swap_add<32>(s[0], s[1]);
+        t = swap_add<16>(t, t);
+        t += dpp_mov<DPP_MIRROR>(t);
+        t += dpp_mov<DPP_HALF_MIRROR>(t);
+        t += dpp_mov<DPP_XOR2>(t);
+        return t + dpp_mov<DPP_XOR1>(t);
+    } else {
+        return wave_col_sums<RW>(s, lane);
     }
 }
 
-// Shape of the resident kernel for B problems of trailing order m on ncu
-// compute units: C columns per thread, R rows and G workgroups per problem,
-// NT threads.  All B G workgroups must be resident at once, one per compute
-// unit, and a thread's R C matrix elements must leave it registers to work
-// with (R C <= 64: 240 of 256 at FP64, nothing spilled).  The fewest rows
-// that fit are the fastest (1024 x 1: R = 8 / 16 / 32 took 4.2 / 4.6 / 5.6 ms).
+// Wave w keeps the rows q G + gi, q = i NW + w (RW of them), all their columns:
+// lane l the columns l + 64 k, k < K.  The words are read once per workgroup and
+// w and a go to LDS, for every wave to form the column.
+// Dynamic LDS: w and a, twice (a column's writes need no barrier
+// behind the last column's reads).
+template <class T>
+constexpr size_t res_rows_lds(int K) { return 4 * (size_t)K * 64 * sizeof(T); }
+
+template <class T, int NW, int RW, int K>
+__global__ __launch_bounds__(64 * NW) void sytrd_resident_rows_kernel(ResArgs<T> g)
+{
+    typedef ResRing<T> Ring;
+    constexpr int R = NW * RW, NT = 64 * NW, CP = (K + NW - 1) / NW, SH = 6 - ilog2<RW>(), ES = (int)sizeof(T), M = 64 * K;
+    constexpr int GS = 2;   // chunks taken together
+    extern __shared__ char smem[];
+    const int n = g.n, m = g.n - g.j0, G = g.G;
+    // (a problem's workgroups on one XCD where G allows it, as in the panel kernel)
+    const int nwg = (int)gridDim.x;
+    const int lin = (nwg % 8 == 0 && (nwg / 8) % G == 0) ? (int)(blockIdx.x & 7) * (nwg / 8) + (int)(blockIdx.x >> 3)
+                                                      : (int)blockIdx.x;
+    const int p = lin / G, gi = lin % G;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    T* A = g.A + (size_t)p * n * n + g.j0 + (size_t)g.j0 * n;   // the trailing matrix, ld n
+    const int bufb = res_buf(G, R) * ES;
+    const __amdgpu_buffer_rsrc_t ring = __builtin_amdgcn_make_buffer_rsrc(
+        g.ring + (size_t)p * RES_RING * res_buf(G, R), 0, RES_RING * bufb, 0x20000);   // (32-bit elements, no stride)
+    T* dd = g.d + (size_t)p * n + g.j0;
+    T* ee = g.e + (size_t)p * n + g.j0;
+    T* tt = g.tau + (size_t)p * n + g.j0;
+    T* lds = reinterpret_cast<T*>(smem);   // 2 x (M of w, M of a), zero where nothing was written
+
+    for (int i = tid; i < 4 * M; i += NT) lds[i] = T(0);
+    // positions of the exchange read by this thread, and their columns (m: none)
+    int col[CP];
+#pragma unroll
+    for (int i = 0; i < CP; i++) {
+        const int pos = tid + i * NT, s = pos % R, c = ((s % RW) * NW + s / RW) * G + pos / R;
+        col[i] = pos < G * R && c < m ? c : m;
+    }
+    // the row this lane publishes, one of the wave's
+    const int il = lane >> SH, rl = (il * NW + wave) * G + gi;
+    const int opub = 2 * ES * (gi * R + wave * RW + il);
+    T a[RW][K], v[K];
+#pragma unroll
+    for (int i = 0; i < RW; i++) {
+        const int r = (i * NW + wave) * G + gi;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const int c = lane + 64 * k;
+            a[i][k] = r < m && c < m ? (c >= r ? A[c + (size_t)r * n] : A[r + (size_t)c * n]) : T(0);
+        }
+    }
+    // column 0 arrives final: into LDS as a (w = 0, v = 0)
+#pragma unroll
+    for (int k = 0; k < K; k++) v[k] = T(0);
+    lds_barrier();
+    for (int c = tid; c < m; c += NT) lds[M + c] = A[c];
+    lds_barrier();
+    T vr_l = 0;   // v of row rl
+    const int rlast = gi < m ? (m - 1 - gi) / G * G + gi : -1, khi = (m - 1) >> 6;
+    T tau = 0, scal = 0, beta = 0, dj = 0;
+    // column j's reflector into A, d, e and tau, by the owner of row j + 1, a
+    // step later: the stores' way to memory is then beside the arithmetic, and
+    // column 0 is overwritten only when every workgroup has loaded its rows
+    auto store_reflector = [&](int j) {
+        if ((j + 1) % G != gi) return;
+        if (tid == 0) {
+            dd[j] = dj;
+            ee[j] = beta;
+            tt[j] = tau;
+        }
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const int c = lane + 64 * k;
+            if (k % NW == wave && c > j && c < m) A[c + (size_t)j * n] = v[k];
+        }
+    };
+    int j = 0;
+    for (; j < m - 1 && rlast > j; j++) {
+        T* lw = lds + (j & 1) * 2 * M;
+        T* la = lw + M;
+        const int kj = j >> 6, k1 = (j + 1) >> 6, l1 = (j + 1) & 63;
+        if (j > 0) {
+            // S and a of the rows from j on (a word that is not wanted is one past
+            // the buffers: no access).  All loads of a pass are issued before
+            // the first is waited for
+            __builtin_amdgcn_s_sleep(RES_WAIT);
+            const int base = (j & (RES_RING - 1)) * bufb, none = RES_RING * bufb;
+            typename Ring::pair pk[CP];
+            int ok[CP];
+#pragma unroll
+            for (int i = 0; i < CP; i++) ok[i] = col[i] >= j && col[i] < m ? base + 2 * ES * (tid + i * NT) : none;
+            for (long spins = 0;; spins++) {
+                asm volatile("" ::: "memory");   // (every pass loads anew)
+#pragma unroll
+                for (int i = 0; i < CP; i++) pk[i] = Ring::get2(ring, ok[i]);
+                bool more = false;
+#pragma unroll
+                for (int i = 0; i < CP; i++) more = more || (ok[i] != none && !Ring::there(pk[i]));
+                if (__builtin_amdgcn_ballot_w64(more) == 0) break;
+                if (res_give_up(spins, g.err, lane)) break;
+            }
+            // (finished columns: zeros)
+#pragma unroll
+            for (int i = 0; i < CP; i++)
+                if (col[i] < m) {
+                    const bool in = col[i] >= j;
+                    const T ak = Ring::second(pk[i]), wk = tau * (scal * Ring::first(pk[i]) + ak);
+                    lw[col[i]] = in ? wk : T(0);
+                    la[col[i]] = in ? ak : T(0);
+                }
+            lds_barrier();
+            store_reflector(j - 1);
+        }
+        // all reads of w and a are issued before the first is used (chunk by
+        // chunk, a read's 130 cycles came twice for each)
+        const T wj = lw[j];
+        const T wl = rl < m ? lw[rl] : T(0), al = rl < m ? la[rl] : T(0);
+        T wv[K], av[K], q = 0;
+#pragma unroll
+        for (int h = 0; h < K; h += GS)
+            if (h + GS > kj && h <= khi) {
+#pragma unroll
+                for (int k = h; k < h + GS; k++) wv[k] = lw[lane + 64 * k];
+            }
+#pragma unroll
+        for (int h = 0; h < K; h += GS)
+            if (h + GS > kj && h <= khi) {
+#pragma unroll
+                for (int k = h; k < h + GS; k++) av[k] = la[lane + 64 * k];
+            }
+        // w^T v, a2 = -tau/2 w^T v
+#pragma unroll
+        for (int h = 0; h < K; h += GS)
+            if (h + GS > kj && h <= khi) {
+                T t = 0;
+#pragma unroll
+                for (int k = h; k < h + GS; k++) t += wv[k] * v[k];
+                q += t;
+            }
+        q = wave_total(q);
+        const T a2 = T(-0.5) * tau * q, a22 = a2 + a2;
+        // the own rows' entries of the column, and the update's factors: a -=
+        // v_r w' + w'_r v = v_r (w + 2 a2 v) + w_r v
+        const T xr_l = al - (wl + a22 * vr_l) - vr_l * wj;
+        T vr[RW], wr[RW];
+#pragma unroll
+        for (int i = 0; i < RW; i++) {
+            vr[i] = read_lane(vr_l, i << SH);
+            wr[i] = read_lane(wl, i << SH);
+        }
+        T nrm = 0, acc[RW], ac[RW], alpha = 0;
+#pragma unroll
+        for (int i = 0; i < RW; i++) acc[i] = ac[i] = T(0);
+#pragma unroll
+        for (int h = 0; h < K; h += GS) {
+            if (h + GS <= kj || h > khi) continue;
+            T wp[GS], x[GS];
+#pragma unroll
+            for (int k = 0; k < GS; k++) {
+                // column j of the updated matrix (v(j) = 1)
+                wp[k] = wv[h + k] + a22 * v[h + k];
+                x[k] = av[h + k] - wp[k] - v[h + k] * wj;
+            }
+            // its head; xt is what is left
+            if (kj >= h && kj < h + GS) {
+#pragma unroll
+                for (int k = 0; k < GS; k++) {
+                    if (h + k != kj) continue;
+                    dj = read_lane(x[k], j & 63);
+                    x[k] = lane == (j & 63) ? T(0) : x[k];
+                }
+            }
+            if (k1 >= h && k1 < h + GS) {
+#pragma unroll
+                for (int k = 0; k < GS; k++) {
+                    if (h + k != k1) continue;
+                    alpha = read_lane(x[k], l1);
+                    x[k] = lane == l1 ? T(0) : x[k];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < RW; i++) {
+                if ((i * NW + wave) * G + gi <= j) continue;
+#pragma unroll
+                for (int k = 0; k < GS; k++) a[i][h + k] -= vr[i] * wp[k] + wr[i] * v[h + k];
+#pragma unroll
+                for (int k = 0; k < GS; k++) acc[i] += a[i][h + k] * x[k];
+            }
+            if (k1 >= h && k1 < h + GS) {
+#pragma unroll
+                for (int k = 0; k < GS; k++) {
+                    if (h + k != k1) continue;
+#pragma unroll
+                    for (int i = 0; i < RW; i++) ac[i] = a[i][h + k];
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < GS; k++) {
+                v[h + k] = x[k];
+                nrm += x[k] * x[k];
+            }
+        }
+        // a(r, j+1) of the row this lane publishes: lane l1 has them all
+        T acl = 0;
+#pragma unroll
+        for (int i = 0; i < RW; i++) {
+            const T t = read_lane(ac[i], l1);
+            acl = il == i ? t : acl;
+        }
+        // publish; the words of two columns ago become free
+        const T s = res_row_sums<RW>(acc, lane);
+        if (j < m - 2) {
+            const int base = ((j + 1) & (RES_RING - 1)) * bufb, old = ((j + 3) & (RES_RING - 1)) * bufb;
+            const bool on = (lane & ((1 << SH) - 1)) == 0 && rl > j && rl < m;
+            __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the last column's clearing stores are complete
+            if (on) Ring::put2(ring, base + opub, Ring::bits(s, acl));
+            if (on) Ring::put2(ring, old + opub, typename Ring::pair(0));
+        } else if (rl == m - 1 && (lane & ((1 << SH) - 1)) == 0) {
+            A[(size_t)(m - 1) * n + m - 1] = acl;   // the last diagonal element (sytrd_finish_kernel moves it to d)
+        }
+        // the reflector
+        nrm = wave_total(nrm);
+        beta = alpha;
+        scal = tau = 0;
+        if (nrm != T(0)) {
+            // |beta| = sqrt(s2) = s2 rsqrt(s2), tau = (beta - alpha) / beta, scal = 1 / (alpha - beta)
+            const T s2 = alpha * alpha + nrm, rs = rsqrt(s2);
+            T b = s2 * rs;
+            b += T(0.5) * rs * fma(-b, b, s2);
+            beta = -copysign(b, alpha);
+            tau = T(1) + fabs(alpha) * rs;
+            scal = res_rcp(alpha - beta);
+        }
+#pragma unroll
+        for (int h = 0; h < K; h += GS) {
+            if (h + GS <= kj || h > khi) continue;
+#pragma unroll
+            for (int k = h; k < h + GS; k++) v[k] = lane + 64 * k == j + 1 ? T(1) : scal * v[k];
+        }
+        vr_l = rl == j + 1 ? T(1) : (rl > j + 1 && rl < m ? scal * xr_l : T(0));
+    }
+    if (j > 0) store_reflector(j - 1);
+}
+
+// Shape of a resident launch for B problems of trailing order m on ncu compute
+// units: R rows and G workgroups per problem, NT threads; C columns per thread,
+// or, where waves have whole rows, K chunks of 64 columns.  All B G workgroups
+// must be resident at once, one per compute unit, and the matrix elements of a
+// thread (R C, or R K 64 / NT) leave it registers to work with (at most 64: 256
+// registers at FP64, nothing spilled).  The fewest rows that fit are the fastest
+// (1024 x 1: R = 8 / 16 / 32 took 4.2 / 4.6 / 5.6 ms), and four waves with whole
+// rows where the registers allow it: eight form the column twice as often.
 struct ResShape {
-    int R = 0, C = 0, G = 0, NT = 0;
+    int R = 0, C = 0, K = 0, G = 0, NT = 0;
 };
 inline ResShape res_shape(int m, int B, int ncu)
 {
@@ -293,14 +702,19 @@ inline ResShape res_shape(int m, int B, int ncu)
         const int G = (m + R - 1) / R;
         if ((long)B * G > ncu) continue;
         s.R = R;
-        s.C = C;
         s.G = G;
-        s.NT = ((m + C - 1) / C + 63) / 64 * 64;
+        if (m <= RES_ROWS_MAX) {
+            s.K = m <= 256 ? 4 : 8;
+            s.NT = R * s.K > 256 ? 512 : 256;
+        } else {
+            s.C = C;
+            s.NT = ((G * R + C - 1) / C + 63) / 64 * 64;   // (G R <= 512 C: R divides 512)
+        }
         return s;
     }
     return s;
 }
-// Largest trailing order the resident kernel takes (0: none).
+// Largest trailing order the resident kernels take (0: none).
 inline int res_max(int B, int ncu)
 {
     int m = 4 * RES_THREADS;
@@ -308,13 +722,22 @@ inline int res_max(int B, int ncu)
     return m >= 2 ? m : 0;
 }
 template <class T>
-const void* res_kernel(int R, int C)
+const void* res_kernel(const ResShape& s)
 {
-    switch (C * 100 + R) {
-        case 108: return (const void*)sytrd_resident_kernel<T, 8, 1>;
-        case 116: return (const void*)sytrd_resident_kernel<T, 16, 1>;
-        case 132: return (const void*)sytrd_resident_kernel<T, 32, 1>;
-        case 164: return (const void*)sytrd_resident_kernel<T, 64, 1>;
+    if (s.K > 0) {
+        switch (s.K * 100 + s.R) {
+            case 408: return (const void*)sytrd_resident_rows_kernel<T, 4, 2, 4>;
+            case 416: return (const void*)sytrd_resident_rows_kernel<T, 4, 4, 4>;
+            case 432: return (const void*)sytrd_resident_rows_kernel<T, 4, 8, 4>;
+            case 464: return (const void*)sytrd_resident_rows_kernel<T, 4, 16, 4>;
+            case 808: return (const void*)sytrd_resident_rows_kernel<T, 4, 2, 8>;
+            case 816: return (const void*)sytrd_resident_rows_kernel<T, 4, 4, 8>;
+            case 832: return (const void*)sytrd_resident_rows_kernel<T, 4, 8, 8>;
+            case 864: return (const void*)sytrd_resident_rows_kernel<T, 8, 8, 8>;
+        }
+        return nullptr;
+    }
+    switch (s.C * 100 + s.R) {
         case 208: return (const void*)sytrd_resident_kernel<T, 8, 2>;
         case 216: return (const void*)sytrd_resident_kernel<T, 16, 2>;
         case 232: return (const void*)sytrd_resident_kernel<T, 32, 2>;
@@ -324,4 +747,9 @@ const void* res_kernel(int R, int C)
         case 416: return (const void*)sytrd_resident_kernel<T, 16, 4>;
     }
     return nullptr;
+}
+template <class T>
+size_t res_lds(int m, const ResShape& s)
+{
+    return s.K > 0 ? res_rows_lds<T>(s.K) : res_lds<T>(m, s.R);
 }

@@ -31,6 +31,33 @@
 // Included by eigen.hip only, inside its namespace.
 #pragma once
 
+// Words of one row's (w, a).
+template <class T>
+constexpr int res_words() { return 2 * (int)(sizeof(T) / 4); }
+
+// Half h of a row's packet (0: w, 1: a).
+__device__ inline void res_put(unsigned long long* q, int h, float x, unsigned ep)
+{
+    const unsigned long long t = (unsigned long long)ep << 32;
+    __hip_atomic_store(q + h, t | __float_as_uint(x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void res_put(unsigned long long* q, int h, double x, unsigned ep)
+{
+    const unsigned long long t = (unsigned long long)ep << 32, b = (unsigned long long)__double_as_longlong(x);
+    __hip_atomic_store(q + 2 * h, t | (b & 0xffffffffull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(q + 2 * h + 1, t | (b >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void res_unpack(const unsigned long long (&x)[2], float& w, float& a)
+{
+    w = __uint_as_float((unsigned)x[0]);
+    a = __uint_as_float((unsigned)x[1]);
+}
+__device__ inline void res_unpack(const unsigned long long (&x)[4], double& w, double& a)
+{
+    w = __longlong_as_double((long long)((x[1] << 32) | (x[0] & 0xffffffffull)));
+    a = __longlong_as_double((long long)((x[3] << 32) | (x[2] & 0xffffffffull)));
+}
+
 constexpr int XP_DW = 4;  // waves that gather exchange D while the others publish B
 constexpr int XP_C = 5;   // rows per thread in exchange A: orders up to XP_C x SY_THREADS
 
