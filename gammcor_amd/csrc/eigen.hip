@@ -881,7 +881,8 @@ __global__ __launch_bounds__(256) void bt_gram_kernel(const T* A, T* G, int nu, 
 // of 16 by the column recurrence (column i of T is -tau_i T(0:i, 0:i)
 // G(0:i, i), diagonal tau_i), then T12 = -T1 U12 T2 from 16 to 32, 64, 128,
 // all in LDS.  The recurrence over 128 columns took 235 us at any order, its
-// serial chain of barriers; this takes about 20.
+// serial chain of barriers; this takes 60 (84 with G's loads, each under its own
+// condition, waited for one by one).
 template <class T>
 __global__ __launch_bounds__(256) void larft_kernel(T* G, const T* tau, int n, int nu, int nbb)
 {
@@ -892,9 +893,21 @@ __global__ __launch_bounds__(256) void larft_kernel(T* G, const T* tau, int n, i
     const int k = q * nbb, kb = min(min(nbb, nu - 1 - k) - o, LT);   // columns of this triangle
     if (kb <= 0) return;
     T* Gb = G + ((size_t)q * gridDim.x + p) * nbb * nbb + o + (size_t)o * nbb;
-    for (int idx = tid; idx < LT * LT; idx += 256) {
-        const int r = idx % LT, c = idx / LT;
-        t[idx] = (r < c && c < kb) ? Gb[r + (size_t)c * nbb] : T(0);
+    // (16 loads at a time, each from a valid place: under their own conditions
+    // they were waited for one by one)
+    constexpr int NL = 16;
+    for (int i0 = tid; i0 < LT * LT; i0 += 256 * NL) {
+        T x[NL];
+#pragma unroll
+        for (int e = 0; e < NL; e++) {
+            const int idx = i0 + 256 * e, r = idx % LT, c = idx / LT;
+            x[e] = Gb[(r < c && c < kb) ? r + (size_t)c * nbb : 0];
+        }
+#pragma unroll
+        for (int e = 0; e < NL; e++) {
+            const int idx = i0 + 256 * e, r = idx % LT, c = idx / LT;
+            t[r + c * LT] = (r < c && c < kb) ? x[e] : T(0);
+        }
     }
     if (tid < LT) ts[tid] = tid < kb ? tau[(size_t)p * n + k + o + tid] : T(0);
     __syncthreads();
@@ -905,8 +918,11 @@ __global__ __launch_bounds__(256) void larft_kernel(T* G, const T* tau, int n, i
         const bool on = tid < LT;
         for (int i = 0; i < LT_BASE; i++) {
             T acc = 0;
-            if (on && r < i)
-                for (int c = r; c < i; c++) acc += tb[r + c * LT] * tb[c + i * LT];
+            if (on && r < i) {
+#pragma unroll
+                for (int c = 0; c < LT_BASE; c++)
+                    if (c < i) acc += c >= r ? tb[r + c * LT] * tb[c + i * LT] : T(0);
+            }
             __syncthreads();
             if (on) {
                 const T ti = ts[bt * LT_BASE + i];
@@ -934,6 +950,7 @@ __global__ __launch_bounds__(256) void larft_kernel(T* G, const T* tau, int n, i
                 const int l0 = pass == 0 ? 0 : r, l1 = pass == 0 ? c + 4 : h;
                 const T* u = t + d + r + (pass == 0 ? d + h : d) * LT;
                 const T* w = t + d + h + (pass == 0 ? d + h + c : d + c) * LT;
+#pragma unroll 4
                 for (int l = l0; l < l1; l++) {
                     T uu[4], ww[4];
 #pragma unroll
@@ -959,7 +976,7 @@ __global__ __launch_bounds__(256) void larft_kernel(T* G, const T* tau, int n, i
     }
     for (int idx = tid; idx < LT * LT; idx += 256) {
         const int r = idx % LT, c = idx / LT;
-        if (r < kb && c < kb) Gb[r + (size_t)c * nbb] = r <= c ? t[idx] : T(0);
+        if (r < kb && c < kb) Gb[r + (size_t)c * nbb] = r <= c ? t[r + c * LT] : T(0);
     }
 }
 
