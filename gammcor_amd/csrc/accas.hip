@@ -441,7 +441,7 @@ size_t ab_scratch_bytes(const AcSystem& s)
                         6 * na2 * na2 * 8});
 }
 
-int assemble_ab01(hipStream_t st, const AcSystem& a, void* scratch, AbPair& out)
+int assemble_ab01(hipStream_t st, const AcSystem& a, void* scratch, AbPair& out, double* later)
 {
     GMC_CHECK(a.N > 0 && a.ndimx > 0, "AB_CAS: empty system");
     const int N = a.N;
@@ -529,6 +529,10 @@ int assemble_ab01(hipStream_t st, const AcSystem& a, void* scratch, AbPair& out)
                            out.m0, out.p1, out.m1);
     }
     GMC_HIP(hipGetLastError());
+    if (later) {
+        GMC_HIP(hipMemcpyAsync(later, d_e, sizeof(double), hipMemcpyDeviceToHost, st));
+        return 0;
+    }
     GMC_HIP(hipMemcpyAsync(&out.ecasscf, d_e, sizeof(double), hipMemcpyDeviceToHost, st));
     GMC_HIP(hipStreamSynchronize(st));
     return 0;

@@ -32,7 +32,9 @@ struct AbPair {
 };
 
 size_t ab_scratch_bytes(const AcSystem& s);
-int assemble_ab01(hipStream_t st, const AcSystem& s, void* scratch, AbPair& out);
+// Waits for the stream and sets out.ecasscf, or with `later` (pinned) only
+// queues its copy to there.
+int assemble_ab01(hipStream_t st, const AcSystem& s, void* scratch, AbPair& out, double* later = nullptr);
 
 // Pair-integral weights of the integrand (acfd.f:4997-5032):
 //   Gw[I,J] = 2 (C_s+C_q)(C_p+C_r) (pr|qs) * [not all four in one geminal]

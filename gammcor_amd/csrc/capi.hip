@@ -214,6 +214,10 @@ int ac_prepare_at(hipStream_t s, int N, int nI, int nA, int ndimx, const double*
     return 0;
 }
 
+// Pinned words of a solve over nalpha points: ECASSCF and the eigensolver's
+// error, then alphas, W and nneg of a batch.
+static size_t ac_pin_bytes(int nalpha) { return 16 + (size_t)nalpha * (2 * sizeof(double) + sizeof(int)); }
+
 // Run the alpha points in batches of `cap` through the ERPA route of `prec`.
 int ac_alpha_batches(hipStream_t s, AcRun& r, int prec, int cap, int nalpha, const double* alphas,
                             double* walpha, double* eig_dev, int* nneg_host)
@@ -222,10 +226,19 @@ int ac_alpha_batches(hipStream_t s, AcRun& r, int prec, int cap, int nalpha, con
     const int nd = r.sys.ndimx;
     cap = std::max(1, std::min(cap, nalpha));
     std::vector<int> nneg(nalpha, 0);
+    // small inputs and results by way of pinned memory and one wait per batch
+    GMC_TRY(st.pin.reserve(ac_pin_bytes(nalpha)));
+    int* const h_err = static_cast<int*>(st.pin.ptr) + 2;
+    double* const h_al = static_cast<double*>(st.pin.ptr) + 2;
+    double* const h_W = h_al + nalpha;
+    int* const h_neg = reinterpret_cast<int*>(h_W + nalpha);
     for (int a0 = 0; a0 < nalpha; a0 += cap) {
         const int B = std::min(cap, nalpha - a0);
         const size_t outb = carve_bytes({B * sizeof(double), (size_t)B * nd * sizeof(double), B * sizeof(int)});
         ErpaOut out;
+        int* d_err = nullptr;        // the plan's error word
+        bool* clear_err = nullptr;
+        std::copy(alphas + a0, alphas + a0 + B, h_al);
         auto bind_out = [&](size_t off) {
             char* base = static_cast<char*>(st.erpaws.ptr) + off;
             out.W = reinterpret_cast<double*>(base);
@@ -246,10 +259,11 @@ int ac_alpha_batches(hipStream_t s, AcRun& r, int prec, int cap, int nalpha, con
                 GMC_TRY(st.erpaws.reserve(align_up(pl.ws_bytes) + outb));
                 bind_out(align_up(pl.ws_bytes));
                 const EigSolveAt factor_eig = st.eig_at(s);
-                GMC_TRY(erpa_batched<T>(s, pl, r.ab, alphas + a0, B, r.Gw, r.wdiag, st.erpaws.ptr, out, nullptr, nullptr,
+                GMC_TRY(erpa_batched<T>(s, pl, r.ab, h_al, B, r.Gw, r.wdiag, st.erpaws.ptr, out, nullptr, nullptr,
                                         nullptr, nullptr, prec == GMC_FP64 ? &factor_eig : nullptr, st.scratch.ptr,
                                         ep->ws_bytes));
-                GMC_TRY(eig_check_error<T>(s, *ep));
+                d_err = ep->err;
+                clear_err = &ep->clear_err;
                 return 0;
             };
             if (prec == GMC_FP64) GMC_TRY(run(double(0)));
@@ -283,7 +297,7 @@ int ac_alpha_batches(hipStream_t s, AcRun& r, int prec, int cap, int nalpha, con
             const size_t mb = erpa_mixed_bytes(nd, B);
             GMC_TRY(st.erpaws.reserve(align_up(mb) + outb));
             bind_out(align_up(mb));
-            GMC_TRY(erpa_batched_mixed(s, *ep, nd, r.ab, alphas + a0, B, r.Gw, r.wdiag, st.erpaws.ptr, mb, out, n_min,
+            GMC_TRY(erpa_batched_mixed(s, *ep, nd, r.ab, h_al, B, r.Gw, r.wdiag, st.erpaws.ptr, mb, out, n_min,
                                            n_max, oa_extend, n_max > n_min ? &resolve : nullptr, half_from, nullptr,
                                            &cluster_eig));
             // rare and as large as an FP64 eigensolver's workspace: not kept
@@ -294,14 +308,19 @@ int ac_alpha_batches(hipStream_t s, AcRun& r, int prec, int cap, int nalpha, con
                 GMC_HIP(hipFree(st.resolve.ptr));
                 st.resolve = Workspace{};
             }
-            GMC_TRY(eig_check_error<float>(s, *ep));
+            d_err = ep->err;
+            clear_err = &ep->clear_err;
         }
-        GMC_HIP(hipMemcpyAsync(walpha + a0, out.W, B * sizeof(double), hipMemcpyDeviceToHost, s));
-        GMC_HIP(hipMemcpyAsync(nneg.data() + a0, out.nneg, B * sizeof(int), hipMemcpyDeviceToHost, s));
+        GMC_HIP(hipMemcpyAsync(h_err, d_err, sizeof(int), hipMemcpyDeviceToHost, s));
+        GMC_HIP(hipMemcpyAsync(h_W, out.W, B * sizeof(double), hipMemcpyDeviceToHost, s));
+        GMC_HIP(hipMemcpyAsync(h_neg, out.nneg, B * sizeof(int), hipMemcpyDeviceToHost, s));
         if (eig_dev)
             GMC_HIP(hipMemcpyAsync(eig_dev + (size_t)a0 * nd, out.eig, (size_t)B * nd * sizeof(double),
                                    hipMemcpyDeviceToDevice, s));
         GMC_HIP(hipStreamSynchronize(s));
+        GMC_TRY(eig_test_error(*h_err, clear_err));
+        std::copy(h_W, h_W + B, walpha + a0);
+        std::copy(h_neg, h_neg + B, nneg.begin() + a0);
     }
     if (nneg_host)
         for (int i = 0; i < nalpha; i++) nneg_host[i] = nneg[i];
@@ -486,7 +505,9 @@ int gmc_acecorr_dev(int prec, int alpha_batch, int nbasis, int ninact, int nact,
     state().sys_valid = false;   // acws is overwritten: drop the host-call system cache
     AcRun r;
     GMC_TRY(ac_prepare(s, nbasis, ninact, nact, ndimx, twono, occ, igem, xone, ure, rdm2act, indn, r));
-    GMC_TRY(assemble_ab01(s, r.sys, r.ab_scratch, r.ab));
+    GMC_TRY(state().pin.reserve(ac_pin_bytes(nalpha)));
+    double* const ecas = static_cast<double*>(state().pin.ptr);
+    GMC_TRY(assemble_ab01(s, r.sys, r.ab_scratch, r.ab, ecas));
     GMC_TRY(integrand_weights(s, r.sys, r.ab.cicoef, r.Gw, r.wdiag));
     std::vector<double> w(nalpha);
     GMC_TRY(ac_alpha_batches(s, r, prec, alpha_batch > 0 ? alpha_batch : 16, nalpha, alphas, w.data(), eig, nneg));
@@ -495,7 +516,7 @@ int gmc_acecorr_dev(int prec, int alpha_batch, int nbasis, int ninact, int nact,
     if (walpha)
         for (int i = 0; i < nalpha; i++) walpha[i] = w[i];
     if (ecorr) *ecorr = e;
-    if (ecasscf) *ecasscf = r.ab.ecasscf;
+    if (ecasscf) *ecasscf = *ecas;   // (the last batch was waited for)
     return 0;
 }
 

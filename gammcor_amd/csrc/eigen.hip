@@ -2249,8 +2249,13 @@ int eig_check_error(hipStream_t s, EigPlan<T>& p)
     int h = 0;
     GMC_HIP(hipMemcpyAsync(&h, p.err, sizeof(int), hipMemcpyDeviceToHost, s));
     GMC_HIP(hipStreamSynchronize(s));
-    if (h != 0) p.clear_err = true;
-    GMC_CHECK(h == 0, "syevd: a workgroup barrier timed out (co-residency lost)");
+    return eig_test_error(h, &p.clear_err);
+}
+
+int eig_test_error(int err, bool* clear)
+{
+    if (err != 0) *clear = true;
+    GMC_CHECK(err == 0, "syevd: a workgroup barrier timed out (co-residency lost)");
     return 0;
 }
 

@@ -101,5 +101,7 @@ int syevd_batched(hipStream_t s, EigPlan<T>& p, T* A, T* w);
 // in any solve since the plan was bound or last checked (the flag is cleared).
 template <class T>
 int eig_check_error(hipStream_t s, EigPlan<T>& p);
+// The same for a plan's error word that was read and its clear_err.
+int eig_test_error(int err, bool* clear);
 
 }  // namespace gmc
