@@ -1047,12 +1047,14 @@ __global__ __launch_bounds__(64) void dc_leaf_kernel(const T* d, const T* e, con
     // cos and sin from h = (a_yy - a_xx) / 2 and g = a_xy: with 1/r =
     // (h^2 + g^2)^(-1/2), cos^2 = (1 + |h|/r) / 2 and sin = sign(h) g / (2 r
     // cos): two reciprocal square roots in a row instead of two square roots
-    // and three divisions
+    // and three divisions.  Entries are at most 1 here: a g below eps^2 is
+    // dropped without a rotation, far below the values' own rounding, and above
+    // it the squares are normal numbers (of subnormal ones cos^2 + sin^2 is not 1)
     auto rotation = [&](int x, int y, T& c, T& sn, T& tn) {
         const T g = A[x][y], h = T(0.5) * (A[y][y] - A[x][x]), r2 = h * h + g * g;
         c = T(1);
         sn = tn = T(0);
-        if (g != T(0) && r2 > T(0)) {
+        if (fabs(g) > Eps<T>::v * Eps<T>::v) {
             const T ir = rsqrt(r2), c2 = T(0.5) + T(0.5) * fabs(h) * ir, ic = rsqrt(c2);
             c = c2 * ic;
             sn = copysign(T(0.5) * ir * ic, h) * g;
