@@ -1801,7 +1801,8 @@ static int eig_layout(EigPlan<T>* p, char* base)
     for (int** v : {&p->perm, &p->lst, &p->lstD, &p->org, &p->rank, &p->rotp, &p->rotj, &p->kcnt, &p->kneg,
                     &p->kpos, &p->kc1, &p->kc2})
         take(*v, B * n * sizeof(int));
-    take(p->bar, (B * G + 1) * BAR_STRIDE * sizeof(unsigned));
+    take(p->bar, ((B * G + 1) * BAR_STRIDE + B) * sizeof(unsigned));
+    p->amax = base ? p->bar + (B * G + 1) * BAR_STRIDE : nullptr;
     take(p->err, 64);
     take(p->fro, B * sizeof(T));
     // padded problems: the reduction runs in Q (free until the divide &
@@ -2019,8 +2020,8 @@ int syevd_batched(hipStream_t s, EigPlan<T>& p, T* A, T* w)
         A = p.Ap;
         w = p.wp;
     }
-    hipLaunchKernelGGL(zero_u32, dim3(((B * G + 1) * BAR_STRIDE + 255) / 256), dim3(256), 0, s, p.bar,
-                       (B * G + 1) * BAR_STRIDE);
+    const int nbar = (B * G + 1) * BAR_STRIDE + B;   // barrier flags, then amax
+    hipLaunchKernelGGL(zero_u32, dim3((nbar + 255) / 256), dim3(256), 0, s, p.bar, nbar);
     if (p.clear_err) {
         hipLaunchKernelGGL(zero_u32, dim3(1), dim3(64), 0, s, (unsigned*)p.err, 16);
         p.clear_err = false;
@@ -2104,12 +2105,17 @@ int syevd_batched(hipStream_t s, EigPlan<T>& p, T* A, T* w)
                 const void* rk = res_kernel<T>(rs);
                 const size_t words = (size_t)B * RES_RING * res_buf(rs.G, rs.R) * (sizeof(T) / 4);   // of 32 bits
                 GMC_CHECK(rk && words * 4 <= (size_t)B * n * 3 * nb * sizeof(T), "syevd: resident shape");
-                ResArgs<T> ra{A, p.d, p.e, p.tau, p.X, p.err, n, k, rs.G};
+                ResArgs<T> ra{A, p.d, p.e, p.tau, p.X, p.amax, p.err, n, k, rs.G};
                 void* rargs[] = {&ra};
                 const size_t rl = res_lds<T>(m, rs);
                 if (!capturing(s)) GMC_HIP(hipFuncSetAttribute(rk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)rl));
-                hipLaunchKernelGGL(zero_u32, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s,
-                                   reinterpret_cast<unsigned*>(p.X), (int)words);
+                if (rs.K > 0)
+                    hipLaunchKernelGGL(zero_u32, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s,
+                                       reinterpret_cast<unsigned*>(p.X), (int)words);
+                else
+                    hipLaunchKernelGGL(res_prepare_kernel<T>, dim3(std::max(1, 512 / B), B), dim3(256), 0, s, ra,
+                                       (int)(words / B), p.amax);
+                GMC_HIP(hipGetLastError());
                 ProfScope ps(s, sizeof(T) == 8 ? "sytrd_resident_f64" : "sytrd_resident_f32", 0.0);
                 GMC_TRY(launch_persistent(rk, dim3(B * rs.G), dim3(rs.NT), rargs, rl, s));
                 break;

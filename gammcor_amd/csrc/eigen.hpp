@@ -47,6 +47,7 @@ struct EigPlan {
     int *rotp = nullptr, *rotj = nullptr, *kcnt = nullptr, *kneg = nullptr;
     int *kpos = nullptr, *kc1 = nullptr, *kc2 = nullptr;   // merge GEMM column grouping
     unsigned* bar = nullptr;
+    unsigned* amax = nullptr;   // largest entry of each problem's resident part
     int* err = nullptr;
     T* fro = nullptr;   // deterministic mode: ||A_b||_F of each problem
     T *Ap = nullptr, *wp = nullptr;   // the padded problems and their eigenvalues (np != n)

@@ -52,6 +52,7 @@ template <class T>
 struct ResArgs {
     T *A, *d, *e, *tau;
     T* ring;                  // per problem RES_RING x res_buf elements, zero on entry
+    const unsigned* amax;     // per problem the largest entry (columns-per-thread layout)
     int* err;
     int n, j0, G;             // order (ld and stride of A, d, e, tau), first column, workgroups per problem
 };
@@ -128,6 +129,40 @@ __device__ inline double res_rcp(double x)
 }
 __device__ inline float res_rcp(float x) { return 1.0f / x; }
 
+// x 2^e, and the exponent of a number from its upper 32 bits without the sign
+// (0 for an infinite or NaN one).
+__device__ inline double res_scale(double x, int e) { return __builtin_amdgcn_ldexp(x, e); }
+__device__ inline float res_scale(float x, int e) { return __builtin_amdgcn_ldexpf(x, e); }
+__device__ inline unsigned res_top(double x) { return (unsigned)((unsigned long long)__double_as_longlong(x) >> 32) & 0x7fffffffu; }
+__device__ inline unsigned res_top(float x) { return __float_as_uint(x) & 0x7fffffffu; }
+template <class T>
+__device__ inline int res_exp(unsigned top)
+{
+    constexpr int MB = sizeof(T) == 8 ? 20 : 23, EMAX = sizeof(T) == 8 ? 0x7ff : 0xff;
+    const int e = (int)(top >> MB);
+    return e == EMAX ? 0 : e - EMAX / 2;
+}
+
+// Zeroes a problem's exchange buffers (words of 32 bits) and finds the largest
+// entry of its trailing matrix (lower triangle; amax zero on entry): 12 us at
+// 2048 x 1 and 20 at 1024 x 8 in FP64, beside 6.8 and 4.1 ms.
+template <class T>
+__global__ __launch_bounds__(256) void res_prepare_kernel(ResArgs<T> g, int words, unsigned* amax)
+{
+    __shared__ unsigned red[4];
+    const int n = g.n, m = g.n - g.j0, p = blockIdx.y;
+    unsigned* ring = reinterpret_cast<unsigned*>(g.ring) + (size_t)p * words;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < words; i += gridDim.x * 256) ring[i] = 0u;
+    const T* A = g.A + (size_t)p * n * n + g.j0 + (size_t)g.j0 * n;
+    unsigned top = 0;
+    for (int c = blockIdx.x; c < m; c += gridDim.x)
+        for (int r = c + threadIdx.x; r < m; r += 256) top = max(top, res_top(A[r + (size_t)c * n]));
+    for (int o = 32; o > 0; o >>= 1) top = max(top, (unsigned)__shfl_xor((int)top, o, 64));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = top;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicMax(&amax[p], max(max(red[0], red[1]), max(red[2], red[3])));
+}
+
 // The sum of the waves' values x[0], x[stride], ...: all loads at once, as a
 // tree (a loop over the waves there are waits for each load: 700 cycles of 8).
 template <class T>
@@ -169,7 +204,11 @@ __device__ inline bool res_give_up(long spins, int* err, int lane)
 // Thread t keeps the columns at the positions t, t + blockDim, ... (at most C)
 // of R rows: what a wave reads of the exchange is contiguous.  The sum of xt^T A
 // xt travels as a share per workgroup: a sum over the column's waves would be a
-// second barrier.
+// second barrier.  It has three factors of the matrix's size, which leave the
+// range long before the two of every other sum here do (FP32: entries of 1e13), so
+// the matrix is reduced as A 2^-ex, ex the exponent of its largest entry, found
+// beforehand (an exchange for it in here cost every column 2-3 % through the
+// registers it takes).
 // Dynamic LDS for a trailing order m (everything twice: a
 // column's writes need no barrier behind the last column's reads).
 template <class T>
@@ -209,6 +248,7 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
     for (int i = tid; i < 2 * RES_WAVES * R; i += NT) part0[i] = T(0);
     lds_barrier();
 
+    const int ex = res_exp<T>(g.amax[p]);
     T a[R][C], v[C], x[C], vown[NCH], wown[NCH];
     int col[C];   // (m: none)
 #pragma unroll
@@ -222,14 +262,14 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
 #pragma unroll
         for (int k = 0; k < C; k++) {
             const int c = col[k];
-            a[q][k] = r < m && c < m ? (c >= r ? A[c + (size_t)r * n] : A[r + (size_t)c * n]) : T(0);
+            a[q][k] = r < m && c < m ? res_scale(c >= r ? A[c + (size_t)r * n] : A[r + (size_t)c * n], -ex) : T(0);
         }
     }
     // column 0 arrives final
 #pragma unroll
     for (int k = 0; k < C; k++) {
         v[k] = T(0);
-        x[k] = col[k] < m ? A[col[k]] : T(0);
+        x[k] = col[k] < m ? res_scale(A[col[k]], -ex) : T(0);
     }
 #pragma unroll
     for (int h = 0; h < NCH; h++) vown[h] = wown[h] = T(0);
@@ -242,8 +282,8 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
         if ((j + 1) % G != gi) return;
         const T* lx = lx0 + (j & 1) * m;
         if (tid == 0) {
-            dd[j] = sc0[4 * (j & 1)];
-            ee[j] = beta;
+            dd[j] = res_scale(sc0[4 * (j & 1)], ex);
+            ee[j] = res_scale(beta, ex);
             tt[j] = tau;
         }
         for (int c = tid; c < m; c += NT)
@@ -401,7 +441,7 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
             scal = res_rcp(alpha - beta);
         }
         if (j == m - 2 && tid == 0)   // the last diagonal element (sytrd_finish_kernel moves it to d)
-            A[(size_t)(m - 1) * n + m - 1] = acol[(m - 1) / G];
+            A[(size_t)(m - 1) * n + m - 1] = res_scale(acol[(m - 1) / G], ex);
 #pragma unroll
         for (int k = 0; k < C; k++) v[k] = col[k] == j + 1 ? T(1) : scal * xt[k];
 #pragma unroll
