@@ -34,8 +34,8 @@
 // Measured, tridiagonalisation alone in FP64: panels and trailing updates -> one
 // exchange per column with two barriers, reflector before publication -> here
 //   order x problems   256 x 64     410 x 8       1024 x 8      1281 x 1      2048 x 1
-//   ms                3.4 1.2 0.78  6.7 1.4 0.97  20.7 4.8 4.04 23.5 5.3 3.75 39.3 9.2 6.79
-// 1.8 us per column at order 85, 2.4 at 410, 2.9 at 1281 (a word's way from one
+//   ms                3.4 1.2 0.82  6.7 1.4 1.00  20.7 4.8 3.96 23.5 5.3 3.86 39.3 9.2 7.09
+// 1.9 us per column at order 85, 2.4 at 410, 3.0 at 1281 (a word's way from one
 // compute unit to another: 0.3 to 0.4 us).
 //
 // Included by eigen.hip only, inside its namespace.
@@ -58,56 +58,68 @@ struct ResArgs {
 };
 
 // Elements of one exchange buffer: (S, a) of every position (gi R + q for row q
-// of workgroup gi), then every workgroup's share of xt^T A xt (to 16 bytes).
+// of workgroup gi; in FP64 every S, then every a), then every workgroup's share
+// of xt^T A xt (to 16 bytes).
 constexpr int res_buf(int G, int R) { return 2 * G * R + (G + 3) / 4 * 4; }
 
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 // Agent-scope words of a buffer (byte offsets): a pair (S, a) and one value.
 // A value's word or half of a pair is never +0 once published.
+//
+// A value counts as there when any of its bits is set, so it must become visible
+// whole: each travels in an aligned access of its own size, 4 or 8 bytes, which
+// is single-copy atomic (the same load and store with the same cache policy that a
+// relaxed agent-scope atomic of that size compiles to).  A 16-byte access is not
+// promised to be: the pair of FP64 is two accesses, S at o and a at o + plane
+// (apart, so that the compiler cannot merge them): as one, 1281 x 1 took
+// 3.78 ms for 3.86, 2048 x 1 6.81 for 7.09, 1024 x 8 4.07 for 3.96.  Of the 8-byte
+// pair of FP32 each half is tested by itself.
 template <class T>
 struct ResRing;
 template <>
 struct ResRing<double> {
     static constexpr int SC1 = 16;   // cache policy: agent scope
-    typedef u32x4 pair;
     typedef u32x2 word;
-    static __device__ inline pair get2(__amdgpu_buffer_rsrc_t r, int o) { return __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, SC1); }
+    struct pair {
+        word s, a;
+    };
     static __device__ inline word get1(__amdgpu_buffer_rsrc_t r, int o) { return __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, SC1); }
-    static __device__ inline void put2(__amdgpu_buffer_rsrc_t r, int o, pair p) { __builtin_amdgcn_raw_buffer_store_b128(p, r, o, 0, SC1); }
     static __device__ inline void put1(__amdgpu_buffer_rsrc_t r, int o, word p) { __builtin_amdgcn_raw_buffer_store_b64(p, r, o, 0, SC1); }
-    static __device__ inline bool there(pair p) { return (p.x | p.y) != 0 && (p.z | p.w) != 0; }
+    static __device__ inline pair get2(__amdgpu_buffer_rsrc_t r, int o, int plane) { return pair{get1(r, o), get1(r, o + plane)}; }
+    static __device__ inline void put2(__amdgpu_buffer_rsrc_t r, int o, int plane, pair p)
+    {
+        put1(r, o, p.s);
+        put1(r, o + plane, p.a);
+    }
     static __device__ inline bool there(word p) { return (p.x | p.y) != 0; }
+    static __device__ inline bool there(pair p) { return there(p.s) && there(p.a); }
     static __device__ inline double val(word p)
     {
         return __longlong_as_double((long long)(((unsigned long long)p.y << 32) | p.x));
     }
-    static __device__ inline double first(pair p) { return val(word{p.x, p.y}); }
-    static __device__ inline double second(pair p) { return val(word{p.z, p.w}); }
+    static __device__ inline double first(pair p) { return val(p.s); }
+    static __device__ inline double second(pair p) { return val(p.a); }
     static __device__ inline word bits(double x)
     {
         const unsigned long long b = (unsigned long long)__double_as_longlong(x);
         const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
         return word{lo, (lo | hi) == 0 ? 0x80000000u : hi};
     }
-    static __device__ inline pair bits(double x, double y)
-    {
-        const word a = bits(x), b = bits(y);
-        return pair{a.x, a.y, b.x, b.y};
-    }
+    static __device__ inline pair bits(double x, double y) { return pair{bits(x), bits(y)}; }
+    static __device__ inline pair clear() { return pair{word(0), word(0)}; }
 };
 template <>
 struct ResRing<float> {
     static constexpr int SC1 = 16;
-    typedef u32x2 pair;
     typedef unsigned word;
-    static __device__ inline pair get2(__amdgpu_buffer_rsrc_t r, int o) { return __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, SC1); }
+    typedef u32x2 pair;
     static __device__ inline word get1(__amdgpu_buffer_rsrc_t r, int o) { return __builtin_amdgcn_raw_buffer_load_b32(r, o, 0, SC1); }
-    static __device__ inline void put2(__amdgpu_buffer_rsrc_t r, int o, pair p) { __builtin_amdgcn_raw_buffer_store_b64(p, r, o, 0, SC1); }
     static __device__ inline void put1(__amdgpu_buffer_rsrc_t r, int o, word p) { __builtin_amdgcn_raw_buffer_store_b32(p, r, o, 0, SC1); }
-    static __device__ inline bool there(pair p) { return p.x != 0 && p.y != 0; }
+    static __device__ inline pair get2(__amdgpu_buffer_rsrc_t r, int o, int) { return __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, SC1); }
+    static __device__ inline void put2(__amdgpu_buffer_rsrc_t r, int o, int, pair p) { __builtin_amdgcn_raw_buffer_store_b64(p, r, o, 0, SC1); }
     static __device__ inline bool there(word p) { return p != 0; }
+    static __device__ inline bool there(pair p) { return p.x != 0 && p.y != 0; }
     static __device__ inline float val(word p) { return __uint_as_float(p); }
     static __device__ inline float first(pair p) { return __uint_as_float(p.x); }
     static __device__ inline float second(pair p) { return __uint_as_float(p.y); }
@@ -117,6 +129,7 @@ struct ResRing<float> {
         return b == 0 ? 0x80000000u : b;
     }
     static __device__ inline pair bits(float x, float y) { return pair{bits(x), bits(y)}; }
+    static __device__ inline pair clear() { return pair(0); }
 };
 
 // 1 / x to rounding level: the hardware's estimate and two Newton steps (the
@@ -231,7 +244,7 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
     const int p = lin / G, gi = lin % G;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, NT = blockDim.x;
     T* A = g.A + (size_t)p * n * n + g.j0 + (size_t)g.j0 * n;   // the trailing matrix, ld n
-    const int bufb = res_buf(G, R) * ES, share = 2 * G * R * ES;
+    const int bufb = res_buf(G, R) * ES, plane = 8 * G * R, share = 2 * G * R * ES;
     const __amdgpu_buffer_rsrc_t ring = __builtin_amdgcn_make_buffer_rsrc(
         g.ring + (size_t)p * RES_RING * res_buf(G, R), 0, RES_RING * bufb, 0x20000);   // (32-bit elements, no stride)
     T* dd = g.d + (size_t)p * n + g.j0;
@@ -310,7 +323,7 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
             typename Ring::pair pk[C], pj = Ring::bits(T(0), T(0));
             typename Ring::word ps[RES_PG];
             bool need[C], needj = true, needs[RES_PG];
-            const int oj = base + 2 * ES * (jg * R + jq);
+            const int oj = base + 8 * (jg * R + jq);
 #pragma unroll
             for (int k = 0; k < C; k++) {
                 pk[k] = Ring::bits(T(0), T(0));
@@ -326,8 +339,8 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
                 asm volatile("" ::: "memory");   // (every pass loads anew)
 #pragma unroll
                 for (int k = 0; k < C; k++)
-                    if (need[k]) pk[k] = Ring::get2(ring, base + 2 * ES * (tid + k * NT));
-                if (needj) pj = Ring::get2(ring, oj);
+                    if (need[k]) pk[k] = Ring::get2(ring, base + 8 * (tid + k * NT), plane);
+                if (needj) pj = Ring::get2(ring, oj, plane);
 #pragma unroll
                 for (int i = 0; i < RES_PG; i++)
                     if (needs[i]) ps[i] = Ring::get1(ring, base + share + ES * (lane + 64 * i));
@@ -416,14 +429,14 @@ __global__ __launch_bounds__(RES_THREADS) void sytrd_resident_kernel(ResArgs<T> 
         if (wave == 0 && j < m - 2) {
             // publish; the words of two columns ago become free
             const int base = ((j + 1) & (RES_RING - 1)) * bufb, old = ((j + 3) & (RES_RING - 1)) * bufb;
-            const int q = lane % R, r = q * G + gi, o = 2 * ES * (gi * R + q);
+            const int q = lane % R, r = q * G + gi, o = 8 * (gi * R + q);
             const T s = res_wave_sum(part + q, R);
             const bool in = r > j && r < m, on = lane < R && in;
             __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the last column's clearing stores are complete
-            if (on) Ring::put2(ring, base + o, Ring::bits(s, acol[q]));
+            if (on) Ring::put2(ring, base + o, plane, Ring::bits(s, acol[q]));
             const T t = res_group_total<R>(in && r > j + 1 ? s * lx[r] : T(0));
             if (lane == 0) Ring::put1(ring, base + share + ES * gi, Ring::bits(t));
-            if (on) Ring::put2(ring, old + o, typename Ring::pair(0));
+            if (on) Ring::put2(ring, old + o, plane, Ring::clear());
             if (lane == 0) Ring::put1(ring, old + share + ES * gi, typename Ring::word(0));
         }
         // the reflector
@@ -499,7 +512,7 @@ __global__ __launch_bounds__(64 * NW) void sytrd_resident_rows_kernel(ResArgs<T>
     const int p = lin / G, gi = lin % G;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     T* A = g.A + (size_t)p * n * n + g.j0 + (size_t)g.j0 * n;   // the trailing matrix, ld n
-    const int bufb = res_buf(G, R) * ES;
+    const int bufb = res_buf(G, R) * ES, plane = 8 * G * R;
     const __amdgpu_buffer_rsrc_t ring = __builtin_amdgcn_make_buffer_rsrc(
         g.ring + (size_t)p * RES_RING * res_buf(G, R), 0, RES_RING * bufb, 0x20000);   // (32-bit elements, no stride)
     T* dd = g.d + (size_t)p * n + g.j0;
@@ -517,7 +530,7 @@ __global__ __launch_bounds__(64 * NW) void sytrd_resident_rows_kernel(ResArgs<T>
     }
     // the row this lane publishes, one of the wave's
     const int il = lane >> SH, rl = (il * NW + wave) * G + gi;
-    const int opub = 2 * ES * (gi * R + wave * RW + il);
+    const int opub = 8 * (gi * R + wave * RW + il);
     T a[RW][K], v[K];
 #pragma unroll
     for (int i = 0; i < RW; i++) {
@@ -567,11 +580,11 @@ __global__ __launch_bounds__(64 * NW) void sytrd_resident_rows_kernel(ResArgs<T>
             typename Ring::pair pk[CP];
             int ok[CP];
 #pragma unroll
-            for (int i = 0; i < CP; i++) ok[i] = col[i] >= j && col[i] < m ? base + 2 * ES * (tid + i * NT) : none;
+            for (int i = 0; i < CP; i++) ok[i] = col[i] >= j && col[i] < m ? base + 8 * (tid + i * NT) : none;
             for (long spins = 0;; spins++) {
                 asm volatile("" ::: "memory");   // (every pass loads anew)
 #pragma unroll
-                for (int i = 0; i < CP; i++) pk[i] = Ring::get2(ring, ok[i]);
+                for (int i = 0; i < CP; i++) pk[i] = Ring::get2(ring, ok[i], plane);
                 bool more = false;
 #pragma unroll
                 for (int i = 0; i < CP; i++) more = more || (ok[i] != none && !Ring::there(pk[i]));
@@ -692,8 +705,8 @@ __global__ __launch_bounds__(64 * NW) void sytrd_resident_rows_kernel(ResArgs<T>
             const int base = ((j + 1) & (RES_RING - 1)) * bufb, old = ((j + 3) & (RES_RING - 1)) * bufb;
             const bool on = (lane & ((1 << SH) - 1)) == 0 && rl > j && rl < m;
             __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the last column's clearing stores are complete
-            if (on) Ring::put2(ring, base + opub, Ring::bits(s, acl));
-            if (on) Ring::put2(ring, old + opub, typename Ring::pair(0));
+            if (on) Ring::put2(ring, base + opub, plane, Ring::bits(s, acl));
+            if (on) Ring::put2(ring, old + opub, plane, Ring::clear());
         } else if (rl == m - 1 && (lane & ((1 << SH) - 1)) == 0) {
             A[(size_t)(m - 1) * n + m - 1] = acl;   // the last diagonal element (sytrd_finish_kernel moves it to d)
         }
