@@ -309,23 +309,49 @@ int abs_factor(hipStream_t s, int n, int B, double* A, double* t0, double* t1, v
     std::vector<int> hb(B);
     int K = 0;
     constexpr double tol = 256 * 2.220446049250313e-16;   // (the residual's rounding floor is a few eps of the norm)
+    // W orthogonalised against V: the next block of V, and into Qt
+    auto next_block = [&]() -> int {
+        for (int pass = 0; pass < 2; pass++) {
+            hipLaunchKernelGGL(vtw_kernel, dim3(m / KB, B), bsk, 0, s, V, nn, n, W, sw, Ct, sc);
+            hipLaunchKernelGGL(skinny_kernel, gsk, bsk, 0, s, V, nn, n, m, Ct, sc, W, sw, nullptr, 0, 1);
+            if (pass == 0)
+                hipLaunchKernelGGL(cholqr_kernel, dim3(B), dim3(1024), 0, s, W, sw, n, W, sw, nullptr, 0, bad);
+            else
+                hipLaunchKernelGGL(cholqr_kernel, dim3(B), dim3(1024), 0, s, W, sw, n, V + (int64_t)m * n, nn, Qt, sw,
+                                   bad);
+        }
+        GMC_HIP(hipGetLastError());
+        m += KB;
+        return 0;
+    };
+    auto breakdown = [&](bool* any) -> int {
+        GMC_HIP(hipMemcpyAsync(hb.data(), bad, B * sizeof(int), hipMemcpyDeviceToHost, s));
+        GMC_HIP(hipStreamSynchronize(s));
+        *any = false;
+        for (int v : hb) *any = *any || v != 0;
+        return 0;
+    };
+    // the caller's eigensolve, and why
+    auto give_up = [&](const char* why) {
+        if (stats) fprintf(stderr, "[gmc] abs_factor: %s in a basis of %d, the eigensolve takes over\n", why, m);
+        return 0;
+    };
     for (int goal = KM_FIRST;;) {
         ProfScope ps(s, "abs_factor_krylov", 0.0);
-        for (; m <= goal; m += KB) {
+        for (;;) {
             // A times the newest block; W starts as that
             hipLaunchKernelGGL(skinny_kernel, gsk, bsk, 0, s, A, nn, n, n, Qt, sw, AV + (int64_t)(m - KB) * n, nn, W, sw,
                                0);
-            if (m == goal) break;
-            for (int pass = 0; pass < 2; pass++) {
-                hipLaunchKernelGGL(vtw_kernel, dim3(m / KB, B), bsk, 0, s, V, nn, n, W, sw, Ct, sc);
-                hipLaunchKernelGGL(skinny_kernel, gsk, bsk, 0, s, V, nn, n, m, Ct, sc, W, sw, nullptr, 0, 1);
-                if (pass == 0)
-                    hipLaunchKernelGGL(cholqr_kernel, dim3(B), dim3(1024), 0, s, W, sw, n, W, sw, nullptr, 0, bad);
-                else
-                    hipLaunchKernelGGL(cholqr_kernel, dim3(B), dim3(1024), 0, s, W, sw, n, V + (int64_t)m * n, nn, Qt,
-                                       sw, bad);
-            }
             GMC_HIP(hipGetLastError());
+            if (m == goal) break;
+            GMC_TRY(next_block());
+            // an exhausted space is noticed here, not after the Ritz problem (at few
+            // sizes: a wait leaves the GPU idle for 40 us)
+            if (m == 8 * KB || m == 16 * KB || m == 32 * KB) {
+                bool any;
+                GMC_TRY(breakdown(&any));
+                if (any) return give_up("breakdown");
+            }
         }
         ps.close();
         // Rayleigh-Ritz: H = V^T (A V)
@@ -339,21 +365,18 @@ int abs_factor(hipStream_t s, int n, int B, double* A, double* t0, double* t1, v
         GMC_TRY(eig(H, theta, m, B, static_cast<char*>(ws) + hbytes, ws_bytes - hbytes));
         th.resize((size_t)B * m);
         GMC_HIP(hipMemcpyAsync(th.data(), theta, th.size() * 8, hipMemcpyDeviceToHost, s));
-        GMC_HIP(hipMemcpyAsync(hb.data(), bad, B * sizeof(int), hipMemcpyDeviceToHost, s));
-        GMC_HIP(hipStreamSynchronize(s));
         K = 0;
         std::vector<int> nb(B, 0);
-        bool broken = false;
+        bool broken;
+        GMC_TRY(breakdown(&broken));
         for (int b = 0; b < B; b++) {
             while (nb[b] < m && th[(size_t)b * m + nb[b]] < 0.0) nb[b]++;
             K = std::max(K, nb[b]);
-            broken = broken || hb[b] != 0 || !std::isfinite(th[(size_t)b * m]) || !std::isfinite(th[(size_t)b * m + m - 1]);
+            broken = broken || !std::isfinite(th[(size_t)b * m]) || !std::isfinite(th[(size_t)b * m + m - 1]);
         }
         K = (K + 1) / 2 * 2;
-        if (broken || K > m / 4) {
-            if (stats) fprintf(stderr, "[gmc] abs_factor: %d pairs below zero in a basis of %d%s\n", K, m, broken ? ", breakdown" : "");
-            return 0;
-        }
+        if (broken) return give_up("breakdown");
+        if (K > m / 4) return give_up("too many pairs below zero");
         double worst = 0.0;
         if (K > 0) {
             // Ritz vectors and their residuals
@@ -370,7 +393,8 @@ int abs_factor(hipStream_t s, int n, int B, double* A, double* t0, double* t1, v
                 const double norm = std::max(std::fabs(th[(size_t)b * m]), std::fabs(th[(size_t)b * m + m - 1]));
                 for (int j = 0; j < nb[b]; j++) {
                     const double r = rs[(size_t)b * K + j] / norm;
-                    worst = !(r <= worst) ? r : worst;
+                    if (!std::isfinite(r)) return give_up("a residual that is not finite");
+                    worst = std::max(worst, r);
                 }
             }
         }
@@ -382,21 +406,13 @@ int abs_factor(hipStream_t s, int n, int B, double* A, double* t0, double* t1, v
             GMC_HIP(hipStreamSynchronize(s));   // (nb leaves the scope)
             break;
         }
-        if (m >= mmax) return 0;
-        // a block gains a factor of 2.2 to 3 here
-        goal = std::min(mmax, m + KB * std::max(4, std::min(24, (int)std::ceil(std::log(worst / tol) / 0.8) + 1)));
+        // a block gains a factor of 2.1 to 2.5 (orders 2236 to 2444, 11 to 40 pairs):
+        // no further where even e each would not do
+        const double gap = std::log(worst / tol);
+        if (m + KB * (int)std::ceil(gap) > mmax) return give_up("no convergence");
+        goal = std::min(mmax, m + KB * std::max(4, std::min(24, (int)std::ceil(gap / 0.8) + 1)));
         // the basis grows on: the newest block's A Q was formed, its successor was not
-        for (int pass = 0; pass < 2; pass++) {
-            hipLaunchKernelGGL(vtw_kernel, dim3(m / KB, B), bsk, 0, s, V, nn, n, W, sw, Ct, sc);
-            hipLaunchKernelGGL(skinny_kernel, gsk, bsk, 0, s, V, nn, n, m, Ct, sc, W, sw, nullptr, 0, 1);
-            if (pass == 0)
-                hipLaunchKernelGGL(cholqr_kernel, dim3(B), dim3(1024), 0, s, W, sw, n, W, sw, nullptr, 0, bad);
-            else
-                hipLaunchKernelGGL(cholqr_kernel, dim3(B), dim3(1024), 0, s, W, sw, n, V + (int64_t)m * n, nn, Qt, sw,
-                                   bad);
-        }
-        GMC_HIP(hipGetLastError());
-        m += KB;
+        GMC_TRY(next_block());
     }
     if (K > 0) {
         // |A| on the lower triangle
@@ -413,8 +429,9 @@ int abs_factor(hipStream_t s, int n, int B, double* A, double* t0, double* t1, v
     for (int v : hb) failed += v != 0;
     if (failed) {
         if (stats) fprintf(stderr, "[gmc] Cholesky route: %d of %d factorisations failed\n", failed, B);
-        return 0;
+        return give_up("a pivot of |A| not above zero");
     }
+    if (stats) fprintf(stderr, "[gmc] abs_factor: |A| factored\n");
     *ok = true;
     return 0;
 }
