@@ -996,6 +996,17 @@ __global__ __launch_bounds__(256) void bt_u_kernel(const T* A, const T* Tall, T*
 }
 
 // ====================================================================== D&C
+// Ascending order of values, a NaN after every number: a total order whatever
+// comes in, so that places in it are a permutation and every output is written.
+template <class T>
+__device__ inline bool val_before(T v, T w) { return w != w ? v == v : v < w; }
+// (v at index u, w at index l, ties in the order of the indices)
+template <class T>
+__device__ inline bool val_before(T v, int u, T w, int l)
+{
+    return w != w ? v == v || u < l : v < w || (v == w && u < l);
+}
+
 // The leaves of the divide & conquer: tridiagonal blocks of at most DC_LEAF
 // rows (leaf[l] .. leaf[l + 1] - 1), their ends less the |e| cut off, solved
 // by cyclic Jacobi in LDS, one wave each.  The 8 x 8 pairs of a round's
@@ -1105,7 +1116,7 @@ __global__ __launch_bounds__(64) void dc_leaf_kernel(const T* d, const T* e, con
         int rank = 0;
         for (int u = 0; u < m; u++) {
             const T v = A[u][u];
-            rank += (v < w || (v == w && u < lane)) ? 1 : 0;
+            rank += val_before(v, u, w, lane) ? 1 : 0;
         }
         lam[(size_t)p * n + s + rank] = ldexp(w, ex);
         T* q = Q + (size_t)p * n * n + s + (size_t)(s + rank) * n;
@@ -1202,9 +1213,6 @@ __global__ __launch_bounds__(256) void dc_prep_kernel(DcArgs a, DcBufs<T> b)
     const T sgn = beta >= T(0) ? T(1) : T(-1);
     const T rs2 = T(0.70710678118654752440);
     T dmax = 0, zmax = 0;
-    // (non-finite values break the places below; every index stays in range)
-    for (int t = tid; t < m; t += 256) perm[t] = t;
-    __syncthreads();
     for (int t = tid; t < m; t += 256) {
         T D = lam[s + t], z;
         int pos;
@@ -1213,7 +1221,7 @@ __global__ __launch_bounds__(256) void dc_prep_kernel(DcArgs a, DcBufs<T> b)
             int lo = 0, hi = m2;   // count right values < D
             while (lo < hi) {
                 int mid = (lo + hi) >> 1;
-                if (lam[s + m1 + mid] < D) lo = mid + 1; else hi = mid;
+                if (val_before(lam[s + m1 + mid], D)) lo = mid + 1; else hi = mid;
             }
             pos = t + lo;
         } else {
@@ -1221,7 +1229,7 @@ __global__ __launch_bounds__(256) void dc_prep_kernel(DcArgs a, DcBufs<T> b)
             int u = t - m1, lo = 0, hi = m1;   // count left values <= D
             while (lo < hi) {
                 int mid = (lo + hi) >> 1;
-                if (lam[s + mid] <= D) lo = mid + 1; else hi = mid;
+                if (!val_before(D, lam[s + mid])) lo = mid + 1; else hi = mid;
             }
             pos = u + lo;
         }
@@ -1550,7 +1558,7 @@ __global__ __launch_bounds__(256) void dc_zhat_kernel(DcArgs a, DcBufs<T> b)
         for (int u0 = 0; u0 < m; u0 += 64) {
             const int u = u0 + lane;
             const T w = u < m ? EV[u] : T(0);
-            r += __popcll(__ballot(u < m && (w < v || (w == v && u < j))));
+            r += __popcll(__ballot(u < m && val_before(w, u, v, j)));
         }
         if (lane == 0) {
             b.rank[po + x] = s + r;
