@@ -2105,9 +2105,9 @@ int syevd_batched(hipStream_t s, EigPlan<T>& p, T* A, T* w)
         unsigned epoch = 0, xepoch = 0;
         for (int k = 0; k < n - 1; k += nb) {
             if (n - k <= p.mres) {
-                // the rest fits in the register files: one resident launch,
-                // 3-5 us per column where a panel's column takes 15 or more
-                // (its two group barriers) at every order that fits
+                // the rest fits in the register files: one resident launch, 2 to
+                // 4 us per column where a panel's column takes 11 or more beside
+                // its SYMV, at every order that fits
                 const int m = n - k;
                 const ResShape rs = res_shape(m, B, p.ncu);
                 const void* rk = res_kernel<T>(rs);

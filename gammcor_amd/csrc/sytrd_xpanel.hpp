@@ -2,8 +2,7 @@
 // algorithm and the row ownership) with its exchanges in self-validating
 // words: what a workgroup tells the others travels as 8-byte words of 32 data
 // bits and the column's epoch (relaxed agent-scope atomics, polled by the
-// reader), as in the resident reduction, instead of plain stores between
-// group barriers.  A barrier costs its fences (write-back and invalidation of
+// reader) instead of plain stores between group barriers.  A barrier costs its fences (write-back and invalidation of
 // the L2, after which the panels are read again), its flag and then the loads
 // of the data: 27 us per column besides the SYMV at every order.
 //
@@ -30,10 +29,6 @@
 //
 // Included by eigen.hip only, inside its namespace.
 #pragma once
-
-// Words of one row's (w, a).
-template <class T>
-constexpr int res_words() { return 2 * (int)(sizeof(T) / 4); }
 
 // Half h of a row's packet (0: w, 1: a).
 __device__ inline void res_put(unsigned long long* q, int h, float x, unsigned ep)

@@ -84,8 +84,6 @@ int transform_plan(int N, TransformPlan* p)
 constexpr int HT_ROWS = 32;   // rows of U (and of Z) per workgroup
 constexpr int HT_NG = 2;      // column blocks of Z a wave forms together, at most
 
-typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-
 // A double at a byte offset of a buffer; past its end it is zero, which is what
 // the padding of N to blocks of 16 needs.
 __device__ inline double buf1(__amdgpu_buffer_rsrc_t r, int o)
@@ -237,8 +235,9 @@ __device__ inline void half_y_some(int left, __amdgpu_buffer_rsrc_t col, __amdgp
 // index j is the larger, one row's 16 columns where k is.  Y lies k-major, rows
 // xor 16 (k & 1): conflict-free both ways.  The panels of a column run on one
 // XCD, whose L2 then reads it once.
-// NB = 2 column blocks at a time leave room for three workgroups per compute
-// unit, whose waits then overlap: whole transform at N = 200 21.5 ms against
+// NB = 2 column blocks at a time leave registers for three workgroups per compute
+// unit (LDS for three up to N = 208, for two above), whose waits then overlap: whole
+// transform at N = 200 21.5 ms against
 // 26.2 with NB = 4 and two workgroups, and against 47.6 as gather, two library
 // products per column and scatter (37 TFLOP/s of a product twice this work; N =
 // 48 0.153 -> 0.083 ms, 160 about 18 -> 7.1).
