@@ -30,18 +30,23 @@
 
 namespace gmc {
 
-// Padded order from which a batching-form group takes the mixed path: on the
-// 64-system workload (padded orders 432-2144, 16 alpha points, up to 256
-// problems per group) every group ran faster in FP64 (20.7 against 19.1
-// solves/s), and single systems gain from order ~3000 on (NBasis=160,
-// NDimX=2664: 0.99x; NBasis=240, NDimX=4524: 1.11x).
+// Padded order from which a batching-form group takes the mixed path.  The line
+// was drawn where single systems began to gain (NBasis=160, NDimX=2664: 0.99x
+// the FP64 speed; NBasis=240, NDimX=4524: 1.11x; below it every group of the
+// 64-system workload ran faster in FP64).  Since the reductions are held in
+// registers and |A+| is factored from its few pairs below zero, FP64 is ahead at
+// both (0.91x, 0.92x): the line no longer divides by speed, it says from where
+// GMC_MIXED gives the mixed path's results.
 constexpr int BATCH_MIXED_MIN = 3000;
 
 namespace {
 
 // Measured on one MI355X (FP64 batches of 16-256 problems, npad 256-1928,
 // tune_batch.py; largest relative misfit 8 %): ms per batch, per padded
-// column, per problem x npad^2 and per problem x npad^3.
+// column, per problem x npad^2 and per problem x npad^3.  The fit is older than
+// the reductions held in registers, which it has no term for: it ranks groupings
+// but overstates times (24 problems padded to 872 and 40 to 488: 106 ms by it, 47
+// measured).
 constexpr double COST_DEFAULT[4] = {1.996, 4.587e-2, 1.084e-6, 4.695e-10};
 
 // One int copied (the eigensolver's barrier flag of a group, kept apart
