@@ -10,7 +10,9 @@ report (GMC_OA_STATS) tells it, and the results on that way.
   of 992): the eigensolve takes over after that one, no second one is tried.
 - Without integrals A+ is diagonal with a few dozen distinct values: the Krylov
   space is exhausted, goes on with rounding noise and breaks down before the basis
-  of the first Ritz problem (832) is full: the eigensolve takes over there."""
+  of the first Ritz problem (832) is full: the eigensolve takes over there.
+- With a NaN among the integrals the basis breaks down at once, the eigensolve
+  takes over and no eigenvalue word is left as it was."""
 import os
 import re
 import sys
@@ -115,3 +117,16 @@ def test_exhausted_space_is_noticed_before_the_ritz_problem(cuda, monkeypatch, c
     (why, basis), = TAKEN_OVER.findall(err)
     assert why == "breakdown" and int(basis) < 832 and not RITZ.search(err)
     assert r["nneg"][0] == 0 and abs(r["ecorr"]) < 1e-12
+
+
+def test_nan_among_the_integrals_breaks_down_and_ends(cuda, monkeypatch, capfd):
+    import torch
+    from gammcor_amd import host
+    monkeypatch.setenv("GMC_OA_STATS", "1")
+    _, d = _device_system(cuda, 150, 8, 8, 8, 450, 0.05, 3)
+    # (p a | q b) with p, q inactive and a, b virtual: one element of A+ and its mirror
+    pair = lambda x, y: max(x, y) * (max(x, y) + 1) // 2 + min(x, y)
+    d.twono[pair(pair(1, 40), pair(3, 90))] = float("nan")
+    r, err = _report(capfd, lambda: host.ACECORR(d, np.array([0.5]), np.array([1.0]), prec=host.GMC_FP64, return_eig=True))
+    assert TAKEN_OVER.findall(err) == [("breakdown", "128")]
+    assert bool(torch.isnan(r["eig"]).any())
